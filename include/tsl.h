@@ -163,7 +163,11 @@ int tsl_map_chunks_to_cells(const int32_t* chunk_pos, const uint32_t* chunk_raw,
 float tsl_likelihood_value(int16_t tsdf_mm, float sigma);
 float tsl_likelihood_init(float sigma);
 
-/* Device bytes held by the map. */
+/* Device bytes of the map as it was loaded: voxels and lookup tables.  A map
+ * that is scored through a class grid (the dense copy of its allocated blocks'
+ * neighbourhood that the scoring kernels read; at most 4 x data_size + 32M
+ * cells of 2 or 4 bytes, below 4 GB) holds that in addition; like a server's
+ * tick buffers it is not charged to a server's budget. */
 int tsl_map_device_bytes(const tsl_map* map, uint64_t* bytes);
 
 int tsl_map_destroy(tsl_map* map);
@@ -262,7 +266,8 @@ int tsl_evaluate_raw_noalloc(tsl_evaluator* ev, const tsl_particle* particles, s
 
 /* Voxel index that CudaSubVoxelMap::getIndex (cuda_sub_voxel_map.tcc:51-137)
  * returns for every (particle, point) pair, row-major [particle][point]
- * (coef.data_size = rejected).  Runs the production lookup on the device; for
+ * (coef.data_size = rejected).  Runs on the device, by the lookup that scores
+ * maps without a class grid (a class grid holds values, not indices); for
  * parity checking.  out has num_particles*num_points entries.  Synchronous. */
 int tsl_trace_indices(tsl_evaluator* ev, const tsl_particle* particles, size_t num_particles,
                       const tsl_point* points, size_t num_points, const float tf_matrix[16],
@@ -282,6 +287,14 @@ int tsl_trace_values(tsl_evaluator* ev, const tsl_particle* particles, size_t nu
  * a multiple of stride.  No counterpart in the reference. */
 int tsl_check_sub_table(float resolution, uint32_t stride, uint64_t* mismatches, uint32_t* entries);
 int tsl_check_magic_divisor(uint32_t divisor, uint32_t stride, uint64_t* mismatches);
+
+/* Self-check of the class grid the scoring kernels read a map through, host
+ * only: the voxel index its tables give for n transformed points t (x, y, z in
+ * map coordinates, |t| < 2^22) -- coef->data_size where init_value is read,
+ * UINT64_MAX where the lookup is left to the exact tiers.  *has_grid = 0 (and
+ * nothing written) if the map has none.  No counterpart in the reference. */
+int tsl_check_class_grid(const tsl_map_coef* coef, const int32_t* grid_occ, const float* t, size_t n,
+                         uint64_t* index, int* has_grid);
 
 /* Pose matrices L[12] (tsdf_evaluator.cpp:102-145) computed on the device
  * with the sin/cos of trig mode `trig` (TSL_TRIG_*). */
@@ -375,7 +388,8 @@ int tsl_filter_restore_async(tsl_filter* f, void* stream);
  * (1, 2 or 4; 0 = automatic; independent gathers in flight) and chunk_len
  * scan points per wavefront (0 = automatic).  Results depend on the tile
  * only through chunk_len (float summation order); k and points_per_lane
- * leave them unchanged.  No counterpart in the reference. */
+ * leave them unchanged, and on a map with a class grid, whose kernel has one
+ * shape, the speed too.  No counterpart in the reference. */
 int tsl_filter_set_tile(tsl_filter* f, int k, int points_per_lane, uint32_t chunk_len);
 
 /* Order in which the particles are evaluated: 0 = caller order, 1 =
@@ -388,8 +402,9 @@ int tsl_filter_set_order(tsl_filter* f, int mode);
 /* How the evaluation finds a block's voxel offset: 0 = the block table in
  * device memory (one gather), 1 = an occupancy bitmap with running counts
  * staged in LDS (no gather; needs offsets in setData order and a table of
- * at most 131072 blocks), -1 = automatic.  Results are identical.  No
- * counterpart in the reference. */
+ * at most 131072 blocks), -1 = automatic.  Results are identical; scoring on
+ * a map with a class grid looks up no blocks.  No counterpart in the
+ * reference. */
 int tsl_filter_set_block_lookup(tsl_filter* f, int mode);
 
 /* Time the candidate evaluation shapes (particle order x block lookup x
@@ -456,8 +471,9 @@ int tsl_batch_destroy(tsl_batch* b);
 /* Tile of the batched evaluation (k particles per wavefront, 1 or 2; points
  * per lane 1, 2 or 4; chunk_len points per chunk, 0 = automatic: 2048, or
  * the whole scan if shorter).  The workgroups of the persistent grid claim
- * work items (4k particles x one chunk) one at a time.  Re-prepares the
- * batch. */
+ * work items (4k particles x one chunk) one at a time; on a map with a class
+ * grid its wavefronts do (2 particles x one chunk, whatever k and
+ * points_per_lane).  Re-prepares the batch. */
 int tsl_batch_set_tile(tsl_batch* b, int k, int points_per_lane, uint32_t chunk_len);
 
 /* Time the batched update (every member, reps launches per candidate on

@@ -1,0 +1,53 @@
+"""The scoring kernels on a class grid: values bit for bit the oracle's and
+weights within 1e-5 of its float64 sum (at most N / 64 + 6 + chunks float
+additions of non-negative terms, 2^-24 each), for palette and float forms, at
+the remainders of particles and points, with lanes in the thin classes below
+the map, lanes and points left to the exact tiers, and matrices out of their
+range."""
+import numpy as np
+import pytest
+
+import oracle_binding as ob
+from test_class_grid import MAPS, _case
+from test_gpu_parity import WEIGHT_RTOL, oracle_values, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("form", ["palette", "float"])
+@pytest.mark.parametrize("name", sorted(MAPS))
+def test_class_grid_values_and_weights(name, form):
+    import tsdf_localization_amd as tsl
+    c, grid, rng = _case(name)
+    c.init_value = 0.0126
+    n = int(c.data_size)
+    data = rng.uniform(0.01, 1.0, 300 if form == "palette" else n).astype(np.float32)
+    data = np.where(rng.uniform(size=n) < 0.5, np.float32(c.init_value), np.resize(data, n)).astype(np.float32)
+    ev = tsl.TSDFEvaluator(tsl.CudaSubVoxelMap(c, grid, data=data))
+    om = ob.OracleMap(c, grid, data)
+    lo = np.array([c.min_x, c.min_y, c.min_z])
+    ext = np.array([c.max_x, c.max_y, c.max_z]) - lo
+    parts = np.zeros((67, 7), np.float32)
+    parts[:, :3] = lo + rng.uniform(-0.3, 1.1, (67, 3)) * ext
+    parts[:, 3:6] = rng.uniform(-3.1, 3.1, (67, 3))
+    parts[:, 6] = 1.0 / 67
+    parts[5, 0] -= 12.0    # thin classes
+    parts[11, 1] -= 40.0   # exact lanes
+    parts[20, 2] += 2e6    # matrix out of range
+    parts[33, 0] = np.inf
+    parts[66, 1] = -3e7
+    pts = (rng.uniform(-1.2, 1.2, (450, 3)) * ext.max()).astype(np.float32)
+    pts[7], pts[100], pts[449] = (7e4, 0, 1), (0, -3e38, 0), (np.inf, 1, 1)
+    tf = np.eye(4, dtype=np.float32)
+    tf[:3, 3] = (0.1, -0.2, 0.3)
+    tf = np.ascontiguousarray(tf.reshape(-1))
+    for P, N in [(1, 1), (2, 64), (3, 65), (2, 127), (67, 128), (5, 129), (66, 191), (67, 450)]:
+        p, q = parts[67 - P:], pts[450 - N:]
+        got = ev.trace_values(p, q, tf)
+        assert np.array_equal(got.view(np.uint32), oracle_values(om, om.trace(p, q, tf)).view(np.uint32)), (P, N)
+        _, w64 = om.evaluate(p, q, tf)
+        assert np.max(rel_err(ev.evaluate_raw(p, q, tf), w64)) <= WEIGHT_RTOL, (P, N)
+    q = pts.copy()
+    q[30, 1] = np.nan
+    got = ev.trace_values(parts, q, tf)
+    assert np.array_equal(got.view(np.uint32), oracle_values(om, om.trace(parts, q, tf)).view(np.uint32))

@@ -103,6 +103,7 @@ _SIGS = {
     "tsl_evaluate_raw_noalloc": (_I, [_P, _P, _S, _P, _S, _P, _P, _P]),
     "tsl_trace_indices": (_I, [_P, _P, _S, _P, _S, _P, _P]),
     "tsl_trace_values": (_I, [_P, _P, _S, _P, _S, _P, _P]),
+    "tsl_check_class_grid": (_I, [ctypes.POINTER(MapCoef), _P, _P, _S, _P, ctypes.POINTER(ctypes.c_int)]),
     "tsl_check_magic_divisor": (_I, [ctypes.c_uint32, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint64)]),
     "tsl_pose_matrices": (_I, [_P, _S, _P, _I, _P]),
     "tsl_evaluator_set_trig": (_I, [_P, _I]),

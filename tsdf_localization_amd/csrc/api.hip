@@ -48,6 +48,14 @@ uint32_t grid_threshold(uint64_t dim, float res)
     return lo;
 }
 
+float lookup_range(const tsl_map_coef& c)
+{
+    // |offset| < R  =>  |trunc| * (1 + up_dim_x + up_dim_2) < 2^31
+    const double lim = 2147483647.0 / (1.0 + (double)c.up_dim_x + (double)c.up_dim_2);
+    const float R = (float)std::min(8388608.0, std::floor(lim));
+    return R < 1.0f ? 1.0f : R;
+}
+
 int launch_set_count(tsl_filter* f, uint32_t n, hipStream_t stream);
 
 int filter_reserve_particles(tsl_filter* f, size_t n)
@@ -367,10 +375,7 @@ static int map_finish(tsl_map* m, const int32_t* grid_occ, const std::vector<flo
     d.gthr_x = fm.gthr_x; d.gthr_y = fm.gthr_y; d.gthr_z = fm.gthr_z;
     d.gneg = fm.gneg_x | (fm.gneg_y << 1) | (fm.gneg_z << 2);
     {
-        // |offset| < R  =>  |trunc| * (1 + up_dim_x + up_dim_2) < 2^31
-        const double lim = 2147483647.0 / (1.0 + (double)c.up_dim_x + (double)c.up_dim_2);
-        float R = (float)std::min(8388608.0, std::floor(lim));
-        if (R < 1.0f) R = 1.0f;
+        const float R = lookup_range(c);
         std::memcpy(&d.range_bits, &R, 4);
         uint64_t neg[8];
         for (int mask = 0; mask < 8; ++mask)
@@ -479,6 +484,11 @@ static int map_finish(tsl_map* m, const int32_t* grid_occ, const std::vector<flo
         // one to three poisoned axes stays below 2^32.  Larger maps send
         // every lane through the recomputation.
         d.carry_limit = 2 * (phys_size + sd3) <= kCarryPoison ? kCarryPoison : 0u;
+    }
+    if (!wide) {
+        TSL_TRY(build_class_grid(m, grid_occ, d.sentinel_code));
+        TSL_TRY(m->dev_copy.reserve(sizeof(DevMap)));
+        TSL_HIP_CHECK(hipMemcpy(m->dev_copy.ptr, &d, sizeof(DevMap), hipMemcpyHostToDevice));
     }
     return TSL_OK;
 }

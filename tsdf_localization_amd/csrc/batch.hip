@@ -63,7 +63,7 @@ int prepare(tsl_batch* b)
     TSL_TRY(b->u0_dev.reserve(sizeof(float) * n));
     TSL_TRY(b->states.reserve(sizeof(FilterState) * n));
     TSL_TRY(b->motions.reserve(sizeof(tsl_motion) * n));
-    uint64_t max_cap = 0, max_items = 0;
+    uint64_t max_cap = 0, rows = 0;
     for (tsl_filter* f : b->filters) {
         const uint64_t need = resample_bound(std::max<size_t>(f->count_bound, f->snapshot_count));
         if (need == 0 || need > 0x7fffffffull)
@@ -113,18 +113,22 @@ int prepare(tsl_batch* b)
         h.stride = (uint32_t)f->capacity;
         h.cap_limit = (uint32_t)f->capacity;
         h.snapshot_count = (uint32_t)f->snapshot_count;
-        const uint64_t per = 4ull * (uint64_t)b->K;  // waves per workgroup x K
-        max_items += (f->capacity + per - 1) / per * t.chunks;
+        rows += (uint64_t)f->capacity * t.chunks;
     }
+    const uint32_t per = batch_item_particles(b->ev->map, b->K, rows);
+    uint64_t max_items = 0;
+    for (const Member& h : b->host_members) max_items += (uint64_t)((h.stride + per - 1) / per) * h.chunks;
     TSL_HIP_CHECK(hipMemcpy(b->members.ptr, b->host_members.data(), sizeof(Member) * n, hipMemcpyHostToDevice));
     BatchLaunch& l = b->launch;
     l.map = b->ev->map;
     l.a_hit = b->ev->a_hit;
+    l.score = score_term_of(b->ev);
     l.members = b->members.as<Member>();
     l.plan = b->plan.as<BatchPlan>();
     l.n = n;
     l.K = b->K;
     l.P = b->P;
+    l.per = per;
     l.max_items = max_items;
     l.max_cap = (uint32_t)max_cap;
     l.max_rs = (uint32_t)max_cap;

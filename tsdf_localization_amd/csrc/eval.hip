@@ -365,9 +365,10 @@ __global__ void k_restore_m(const Member* __restrict__ members)
 }
 
 // Work plan of a batched evaluation: member f owns items [prefix[f],
-// prefix[f+1]), groups x chunks of them in (particle group, chunk) order;
+// prefix[f+1]), groups (of `per` particles) x chunks of them in (particle
+// group, chunk) order;
 // the item counter starts at zero.
-__global__ __launch_bounds__(1024) void k_batch_plan(const Member* __restrict__ members, uint32_t n, uint32_t K,
+__global__ __launch_bounds__(1024) void k_batch_plan(const Member* __restrict__ members, uint32_t n, uint32_t per,
                                                      BatchPlan* __restrict__ plan)
 {
     __shared__ uint32_t wsum[16];
@@ -375,7 +376,6 @@ __global__ __launch_bounds__(1024) void k_batch_plan(const Member* __restrict__ 
     uint32_t items = 0;
     if (f < n) {
         const Member& m = members[f];
-        const uint32_t per = kWaves * K;
         items = m.N ? (m.st->count + per - 1) / per * m.chunks : 0u;
     }
     // block exclusive scan
@@ -434,6 +434,7 @@ Tile choose_tile(const tsl_filter* f, size_t P, size_t N)
     t.P = f->tile_p ? f->tile_p : 1;
     t.order = f->order_mode >= 0 ? f->order_mode : (P >= 8192 ? 1 : 0);
     t.rank = f->rank_mode >= 0 ? f->rank_mode : 1;
+    t.grid = f->ev->map->grid.ready != 0;
     const size_t groups = (P + t.K - 1) / t.K;
     size_t len;
     if (f->tile_chunk) {
@@ -479,6 +480,8 @@ int launch_eval_kernel(const Tile& tile, const tsl_filter* f, size_t P, size_t N
     const size_t groups = (P + tile.K - 1) / tile.K;
     const size_t items = (groups + kWaves - 1) / kWaves * tile.chunks;
     if (items > 0x7fffffffull) return set_error(TSL_ERR_UNSUPPORTED, "evaluation grid too large");
+    // (the class grid holds values, not the reference's indices)
+    if (kMode != 1 && tile.grid) return launch_grid(kMode, f, tile, P, N, stream, partial, trace_out);
     const dim3 grid((unsigned)items);
     const bool rank = tile.rank && map->dev.occ_nwords != 0;
     const size_t lds = lds_bytes(map->dev, rank);
@@ -625,7 +628,8 @@ int autotune_tile(tsl_filter* f, hipStream_t stream, int reps, int* best_order, 
     const int ps[3] = {1, 2, 4};
     const uint32_t div[5] = {0, 1, 2, 4, 8};
     int rc = TSL_OK;
-    const int ranks = f->ev->map->dev.occ_nwords ? 2 : 1;
+    // a class grid has neither a block table nor a rank table to choose
+    const int ranks = !f->ev->map->grid.ready && f->ev->map->dev.occ_nwords ? 2 : 1;
     for (int order = 0; order < 2 && rc == TSL_OK; ++order) {
         f->order_mode = order;
         Tile pt = choose_tile(f, P, N);
@@ -784,6 +788,7 @@ namespace {
 
 int dispatch_eval_batch(const BatchLaunch& b, hipStream_t stream, uint32_t* grid_out)
 {
+    if (b.map->grid.ready) return launch_grid_batch(b, stream, grid_out);
     switch (b.K * 8 + b.P) {
     case 9: return launch_eval_batch_tile_1_1(b, stream, grid_out);
     case 10: return launch_eval_batch_tile_1_2(b, stream, grid_out);
@@ -796,6 +801,13 @@ int dispatch_eval_batch(const BatchLaunch& b, hipStream_t stream, uint32_t* grid
 }
 
 }  // namespace
+
+uint32_t batch_item_particles(const tsl_map* map, int K, uint64_t rows)
+{
+    return map->grid.ready ? grid_item_particles(rows) : (uint32_t)(kWaves * K);
+}
+
+uint32_t batch_group_items(const tsl_map* map) { return map->grid.ready ? grid_threads(map->grid) / 64 : 1u; }
 
 int batch_grid(const BatchLaunch& b, uint32_t* grid) { return dispatch_eval_batch(b, nullptr, grid); }
 
@@ -814,7 +826,8 @@ int launch_batch_update(const BatchLaunch& b, hipStream_t stream)
     const unsigned gx = (b.max_cap + 255) / 256 ? (b.max_cap + 255) / 256 : 1;
     hipLaunchKernelGGL(k_pose_m, dim3(gx, b.n), dim3(256), 0, stream, b.members);
     TSL_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(1024), 0, stream, b.members, b.n, (uint32_t)b.K, b.plan);
+    hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(1024), 0, stream, b.members, b.n,
+                       b.per, b.plan);
     TSL_HIP_CHECK(hipGetLastError());
     if (b.grid == 0) return set_error(TSL_ERR_INVALID_ARGUMENT, "batch grid not sized");
     TSL_TRY(dispatch_eval_batch(b, stream, nullptr));

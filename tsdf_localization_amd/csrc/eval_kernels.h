@@ -15,6 +15,7 @@
 
 #include "tsl_lookup.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace tsl {
@@ -594,34 +595,31 @@ int launch_eval_flags(bool u24, bool brick, bool rank, dim3 grid, size_t lds, hi
 #undef TSL_EVAL_ARGS
 }
 
-// stream == nullptr && grid_out: report the persistent grid size only.
 __global__ void k_batch_claims_reset(BatchPlan* __restrict__ plan)
 {
     if (threadIdx.x < kPlanXcds) plan->next[threadIdx.x * 32] = 0;
 }
 
-template <int K, int kP, bool kU24, bool kBrick, bool kRank, bool kWide = false, bool kF32 = false>
-int launch_eval_batch_t(const BatchLaunch& b, hipStream_t stream, uint32_t* grid_out)
+// Workgroups of a persistent kernel: as many as are resident, no more than
+// `need`, a multiple of the XCDs.
+int resident_groups(const void* kernel, int threads, size_t lds, int device, uint64_t need, uint32_t* groups)
 {
-    constexpr auto kernel = batch_kernel<K, kP, kU24, kBrick, kRank, kWide, kF32>();
-    TSL_CHECK_PALETTE_AT_ZERO(kernel);
-    const size_t lds = lds_bytes(b.map->dev, kRank);
-    if (grid_out) {
-        int per_cu = 0;
-        TSL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(kernel), kBlock,
-            lds));
-        if (per_cu < 1) per_cu = 1;
-        int cus = 0;
-        TSL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b.map->device));
-        uint64_t grid = (uint64_t)per_cu * (uint64_t)cus;
-        const uint64_t need = (b.max_items + kXcds - 1) / kXcds * kXcds;
-        if (grid > need) grid = need;
-        grid = (grid + kXcds - 1) / kXcds * kXcds;
-        if (grid < kXcds) grid = kXcds;
-        *grid_out = (uint32_t)grid;
-        return TSL_OK;
-    }
+    int per_cu = 0;
+    TSL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds));
+    if (per_cu < 1) per_cu = 1;
+    int cus = 0;
+    TSL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    uint64_t grid = std::min<uint64_t>((uint64_t)per_cu * (uint64_t)cus, (need + kXcds - 1) / kXcds * kXcds);
+    grid = (grid + kXcds - 1) / kXcds * kXcds;
+    *groups = (uint32_t)std::max<uint64_t>(grid, kXcds);
+    return TSL_OK;
+}
+
+// One launch for all items, or one per slice of them with the claim counters
+// reset in between.
+template <typename Launch>
+int launch_slices(const BatchLaunch& b, hipStream_t stream, Launch&& launch)
+{
     const uint64_t slice = b.slice_items ? b.slice_items : (uint64_t)0xffffffffu;
     const uint64_t end = b.slice_items ? std::min<uint64_t>(b.max_items, 0xffffffffull) : 1;
     for (uint64_t i0 = 0; i0 < end; i0 += slice) {
@@ -629,12 +627,25 @@ int launch_eval_batch_t(const BatchLaunch& b, hipStream_t stream, uint32_t* grid
             hipLaunchKernelGGL(k_batch_claims_reset, dim3(1), dim3(64), 0, stream, b.plan);
             TSL_HIP_CHECK(hipGetLastError());
         }
-        hipLaunchKernelGGL(kernel, dim3(b.grid), dim3(kBlock), lds,
-                           stream, b.map->dev, b.members, b.plan, b.a_hit, (uint32_t)i0,
-                           (uint32_t)std::min<uint64_t>(slice, 0xffffffffu));
+        launch((uint32_t)i0, (uint32_t)std::min<uint64_t>(slice, 0xffffffffu));
         TSL_HIP_CHECK(hipGetLastError());
     }
     return TSL_OK;
+}
+
+// grid_out: report the persistent grid size only.
+template <int K, int kP, bool kU24, bool kBrick, bool kRank, bool kWide = false, bool kF32 = false>
+int launch_eval_batch_t(const BatchLaunch& b, hipStream_t stream, uint32_t* grid_out)
+{
+    constexpr auto kernel = batch_kernel<K, kP, kU24, kBrick, kRank, kWide, kF32>();
+    TSL_CHECK_PALETTE_AT_ZERO(kernel);
+    const size_t lds = lds_bytes(b.map->dev, kRank);
+    if (grid_out)
+        return resident_groups(reinterpret_cast<const void*>(kernel), kBlock, lds, b.map->device, b.max_items, grid_out);
+    return launch_slices(b, stream, [&](uint32_t item0, uint32_t count) {
+        hipLaunchKernelGGL(kernel, dim3(b.grid), dim3(kBlock), lds, stream, b.map->dev, b.members, b.plan, b.a_hit,
+                           item0, count);
+    });
 }
 
 template <int K, int kP>

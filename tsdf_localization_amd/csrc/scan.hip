@@ -61,16 +61,24 @@ __global__ void k_morton(const tsl_point* __restrict__ in, uint32_t n, uint64_t*
     vals[i] = i;
 }
 
-// Sorted point j = input point perm[j], with its constant score term
-// (tsdf_evaluator.cpp:56-65): |p|^2 evaluated as the reference does.
+// A point with its constant score term (tsdf_evaluator.cpp:56-65): |p|^2
+// evaluated as the reference does.  mark: NaN instead for points that the
+// class-grid kernels leave to the exact tiers.
+__device__ __forceinline__ float4 scored_point(const tsl_point& p, const ScoreTerm& sc, int mark)
+{
+    const float d2 = p.x * p.x + p.y * p.y + p.z * p.z;
+    float w = d2 < sc.max_range_squared ? sc.range_term : sc.a_max;
+    if (mark && !(fabsf(p.x) < kTamePoint && fabsf(p.y) < kTamePoint && fabsf(p.z) < kTamePoint)) w = __builtin_nanf("");
+    return make_float4(p.x, p.y, p.z, w);
+}
+
+// Sorted point j = input point perm[j].
 __global__ void k_prep_sorted(const tsl_point* __restrict__ in, const uint32_t* __restrict__ perm, uint32_t n,
-                              float range_term, float a_max, float mr2, float4* __restrict__ out)
+                              ScoreTerm sc, int mark, float4* __restrict__ out)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
-    const tsl_point p = in[perm[j]];
-    const float d2 = p.x * p.x + p.y * p.y + p.z * p.z;
-    out[j] = make_float4(p.x, p.y, p.z, d2 < mr2 ? range_term : a_max);
+    out[j] = scored_point(in[perm[j]], sc, mark);
 }
 
 // Evaluation order of the particles: a counting sort into Morton-ordered
@@ -486,8 +494,7 @@ int launch_prep_points(tsl_filter* f, hipStream_t stream)
                                                      f->perm.as<uint32_t>(), (int)n, 0, 63, stream));
     const tsl_evaluator* ev = f->ev;
     hipLaunchKernelGGL(k_prep_sorted, dim3(g), dim3(256), 0, stream, f->points_in.as<tsl_point>(),
-                       f->perm.as<uint32_t>(), n, ev->range_term, ev->a_max, ev->max_range_squared,
-                       f->points.as<float4>());
+                       f->perm.as<uint32_t>(), n, score_term_of(ev), (int)ev->map->grid.ready, f->points.as<float4>());
     TSL_HIP_CHECK(hipGetLastError());
     return TSL_OK;
 }
@@ -497,7 +504,7 @@ namespace {
 // Sorted position i of scan blockIdx.y: the point and its score constant,
 // as k_prep_sorted writes them for one filter.
 __global__ void k_prep_sorted_seg(const tsl_point* __restrict__ in, const uint32_t* __restrict__ off,
-                                  const uint32_t* __restrict__ sorted_idx, float range_term, float a_max, float mr2,
+                                  const uint32_t* __restrict__ sorted_idx, ScoreTerm sc, int mark,
                                   const ScanDest* __restrict__ dst)
 {
     const uint32_t r = blockIdx.y;
@@ -505,9 +512,7 @@ __global__ void k_prep_sorted_seg(const tsl_point* __restrict__ in, const uint32
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t src = sorted_idx[b + i];
-    const tsl_point p = in[src];
-    const float d2 = p.x * p.x + p.y * p.y + p.z * p.z;
-    dst[r].points[i] = make_float4(p.x, p.y, p.z, d2 < mr2 ? range_term : a_max);
+    dst[r].points[i] = scored_point(in[src], sc, mark);
     dst[r].perm[i] = src - b;
 }
 
@@ -563,7 +568,7 @@ int launch_prep_points_batch(const tsl_evaluator* ev, const tsl_point* pts, cons
     TSL_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, seg, seg + total, vals + total, vals,
                                                      (int)total, 0, bits, stream));
     hipLaunchKernelGGL(k_prep_sorted_seg, dim3((max_count + 255) / 256, n), dim3(256), 0, stream, pts, off, vals,
-                       ev->range_term, ev->a_max, ev->max_range_squared, dst);
+                       score_term_of(ev), (int)ev->map->grid.ready, dst);
     TSL_HIP_CHECK(hipGetLastError());
     return TSL_OK;
 }

@@ -228,8 +228,10 @@ int dispatch(tsl_server* s, Slot* sl)
 {
     hipStream_t st = s->stream[sl->cls];
     const uint32_t n = (uint32_t)sl->reqs.size();
-    uint64_t max_items = 0;
+    uint64_t rows = 0;
     uint32_t max_cap = 0;
+    const uint64_t at_once = batch_group_items(s->ev->map);  // items a workgroup works on at a time
+    const uint64_t group_waves = s->ev->map->grid.ready ? at_once : 4;
     // every scan of the tick: one upload, one preparation
     uint32_t total = 0, max_np = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -308,32 +310,42 @@ int dispatch(tsl_server* s, Slot* sl)
         h.cap_limit = (uint32_t)f->capacity;
         sl->u0_host[i] = pd.req.u0;
         sl->motions_host[i] = pd.req.motion;
-        max_items += (f->capacity + 4 * s->K[sl->cls] - 1) / (4 * s->K[sl->cls]) * chunks;
+        rows += (uint64_t)f->capacity * chunks;
         max_cap = std::max<uint32_t>(max_cap, (uint32_t)f->capacity);
     }
     TSL_HIP_CHECK(hipMemcpyAsync(sl->members.ptr, sl->members_host, sizeof(Member) * n, hipMemcpyHostToDevice, st));
     TSL_HIP_CHECK(hipMemcpyAsync(sl->u0.ptr, sl->u0_host, sizeof(float) * n, hipMemcpyHostToDevice, st));
     TSL_HIP_CHECK(hipMemcpyAsync(sl->motions.ptr, sl->motions_host, sizeof(tsl_motion) * n, hipMemcpyHostToDevice, st));
+    const uint32_t per = batch_item_particles(s->ev->map, s->K[sl->cls], rows);
+    uint64_t max_items = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const Member& h = sl->members_host[i];
+        max_items += (uint64_t)((h.stride + per - 1) / per) * h.chunks;
+    }
     BatchLaunch l;
     l.map = s->ev->map;
     l.a_hit = s->ev->a_hit;
+    l.score = score_term_of(s->ev);
     l.members = sl->members.as<Member>();
     l.plan = sl->plan.as<BatchPlan>();
     l.n = n;
     l.K = s->K[sl->cls];
     l.P = s->P[sl->cls];
     l.rank = true;
+    l.per = per;
     l.max_items = max_items;
     l.max_cap = max_cap;
     l.max_rs = max_cap;
-    // a bulk tick leaves one workgroup slot per compute unit to the other
-    // stream and evaluates in slices of about slice_pairs pairs
-    const int pc = s->per_cu[sl->cls];
-    const int per_cu = (sl->cls == 1 && s->slice_pairs)
-                           ? std::max(1, pc - (int)std::min<uint32_t>(s->reserved_per_cu, (uint32_t)pc))
-                           : pc;
-    uint64_t grid = (uint64_t)per_cu * (uint64_t)s->cus;
-    const uint64_t need = (max_items + 7) / 8 * 8;
+    // a bulk tick leaves the room of reserved_per_cu four-wavefront
+    // workgroups per compute unit, and at most all but one workgroup of
+    // each, to the other stream and evaluates in slices of about
+    // slice_pairs pairs
+    uint64_t grid = (uint64_t)s->per_cu[sl->cls] * (uint64_t)s->cus;
+    if (sl->cls == 1 && s->slice_pairs) {
+        const uint64_t keep = (uint64_t)s->reserved_per_cu * 4 * (uint64_t)s->cus / group_waves;
+        grid = std::max<uint64_t>((uint64_t)s->cus, grid - std::min(grid, keep));
+    }
+    const uint64_t need = ((max_items + at_once - 1) / at_once + 7) / 8 * 8;
     if (grid > need) grid = need;
     grid = std::max<uint64_t>(8, (grid + 7) / 8 * 8);
     l.grid = (uint32_t)grid;
@@ -341,8 +353,8 @@ int dispatch(tsl_server* s, Slot* sl)
         uint64_t pairs_per_item = 0;
         for (uint32_t i = 0; i < n; ++i)
             pairs_per_item =
-                std::max<uint64_t>(pairs_per_item, (uint64_t)4 * s->K[1] * sl->members_host[i].chunk_len);
-        l.slice_items = std::max<uint64_t>(grid, s->slice_pairs / std::max<uint64_t>(pairs_per_item, 1));
+                std::max<uint64_t>(pairs_per_item, (uint64_t)per * sl->members_host[i].chunk_len);
+        l.slice_items = std::max<uint64_t>(grid * at_once, s->slice_pairs / std::max<uint64_t>(pairs_per_item, 1));
     }
     TSL_TRY(launch_motion_members(l.members, sl->motions.as<tsl_motion>(), n, max_cap, st));
     for (uint32_t i = 0; i < n; ++i) {

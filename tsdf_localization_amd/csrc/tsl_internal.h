@@ -189,8 +189,65 @@ struct DevMap {
     uint32_t f32;                     // 1: float form (more distinct values than the palette holds)
 };
 
+// Class grid of a map (class_grid.hip): what the scoring kernels of
+// grid_eval.hip read.
+struct DevGrid {
+    const AxisEntry* axis;     // bucket table of x, then y, then z: class boundary (float bits), address terms below / from it
+    const uint8_t* bits;       // bitmap: granule i (2^shift bytes of cells) holds a value other than init_value
+    const void* cells;         // dense array: LDS addresses of the values (bits_bytes + 4 palette index), or, float form, the values
+    const float* palette;      // the map's palette, then the NaN of the lanes of the exact tiers
+    float scale;               // buckets per metre
+    float off[3], top[3];      // bucket of t: fma(t, scale, off), at most top (and at least kGridMagic)
+    uint32_t first[3];         // an axis's first entry
+    uint32_t entries, bits_bytes, shift, palette_size;
+    uint32_t init_code;        // cell of init_value
+    float init;
+    uint32_t ready;            // 0: the map has no class grid
+};
+constexpr float kGridMagic = 12582912.0f;  // 1.5 * 2^23, bucket 0
+// Scan points at or past this (or not finite) carry a NaN score term on a map
+// with a class grid: the kernels take their pairs through the exact tiers.
+constexpr float kTamePoint = 65536.0f;
+// LDS bytes of the scoring kernels on a class grid: bitmap, palette, bucket tables.
+constexpr size_t grid_lds_bytes(const DevGrid& g)
+{
+    return g.bits_bytes + 16 * ((g.palette_size + 3ull) / 4) + 16ull * g.entries;
+}
+// Particles of a wavefront's item on a class grid, for particles x chunks in
+// all: two, which the kernel works on at a time, or as many more as keep the
+// items below 2^31.
+constexpr uint32_t grid_item_particles(uint64_t rows)
+{
+    uint32_t per = 2;
+    while (rows / per >= (1ull << 30)) per *= 2;
+    return per;
+}
+// Threads of a workgroup: the fewest wavefronts (4, 8 or 16) that keep as many
+// as possible resident on a CU (160 KB of LDS, 32 wavefronts).
+constexpr uint32_t grid_threads(const DevGrid& g)
+{
+    uint32_t best = 256, waves = 0;
+    for (uint32_t t = 256; t <= 1024; t *= 2) {
+        const size_t fit = (160u << 10) / grid_lds_bytes(g);
+        const uint32_t n = (uint32_t)(fit < 2048u / t ? fit : 2048u / t) * (t / 64);
+        if (n > waves) {
+            waves = n;
+            best = t;
+        }
+    }
+    return best;
+}
+constexpr size_t kGridLdsBudget = 80 << 10;  // two workgroups of 16 wavefronts on a CU's 160 KB
+
 // Smallest u in [0, 2^23] with trunc(fl(fl(u)/res)) >= dim; host IEEE division.
 uint32_t grid_threshold(uint64_t dim, float res);
+// Bound R of |offset| that keeps every block index of the 32-bit tiers in int32.
+float lookup_range(const tsl_map_coef& c);
+
+// class_grid.hip: the class grid of an uploaded map (map->dev complete), or
+// grid.ready == 0 where the map has none (wide maps, extents or tables past
+// the LDS budget or 32-bit addresses).
+int build_class_grid(tsl_map* m, const int32_t* grid_occ, uint32_t init_code);
 
 // tables.hip
 int build_sub_table(float res, SubTable* out);
@@ -298,7 +355,10 @@ struct tsl_map {
     tsl_map_coef coef{};
     tsl::DevBuf grid_occ, codes, palette, sub_tab, neg_tab, full, occ_words, axis_tab;
     tsl::DevBuf slots;       // wide maps: uint32 block slots (grid_occ unused)
+    tsl::DevBuf grid_axis, grid_bits, grid_cells, grid_palette;  // class grid
+    tsl::DevBuf dev_copy;    // dev, for the class grid's exact lanes
     tsl::DevMap dev{};
+    tsl::DevGrid grid{};
 };
 
 struct tsl_evaluator {
@@ -383,6 +443,7 @@ struct Tile {
     int P;               // points per lane per iteration
     int order;           // 1: particles evaluated in spatial order
     int rank;            // 1: block offsets from the LDS occupancy-rank table (when the map has one)
+    int grid;            // 1: on the map's class grid (K, P and rank do not apply)
     uint32_t chunk_len;
     uint32_t chunks;
 };
@@ -433,15 +494,26 @@ void pose_from_stats(const double* st, tsl_pose* pose);
 // Map a FilterState status to the library's error (TSL_OK if none).
 int status_error(uint32_t status);
 
+// The point term of the score, for points whose prepared one is NaN.
+struct ScoreTerm {
+    float range_term, a_max, max_range_squared;
+};
+inline ScoreTerm score_term_of(const tsl_evaluator* ev)
+{
+    return ScoreTerm{ev->range_term, ev->a_max, ev->max_range_squared};
+}
+
 // Batched update (eval.hip)
 struct BatchLaunch {
     const tsl_map* map = nullptr;
     float a_hit = 0.9f;
+    ScoreTerm score{};
     Member* members = nullptr;   // device array [n]
     BatchPlan* plan = nullptr;   // device
     uint32_t n = 0;
     int K = 1, P = 1;
     uint64_t max_items = 0;      // upper bound of the evaluation items over all members
+    uint32_t per = 0;            // particles of an item (batch_item_particles)
     uint32_t max_cap = 0;        // largest member capacity (grid bound of the per-particle kernels)
     uint32_t max_rs = 0;         // largest resampling output room
     uint32_t grid = 0;           // persistent evaluation grid (multiple of the XCD count)
@@ -449,6 +521,18 @@ struct BatchLaunch {
     uint64_t slice_items = 0;    // evaluation items per launch (0: one launch for all)
 };
 int launch_batch_update(const BatchLaunch& b, hipStream_t stream);
+// Particles of an item of the batched evaluation (x one chunk) with K particles
+// per wavefront and `rows` particles x chunks over all members, and the items
+// a workgroup works on at a time.
+uint32_t batch_item_particles(const tsl_map* map, int K, uint64_t rows);
+uint32_t batch_group_items(const tsl_map* map);
+// Scoring (mode 0) or value trace (mode 2) on a map's class grid (grid_eval.hip).
+// init, once per map on its device: the kernels may need more dynamic LDS than
+// the runtime grants unasked, and read their tables from LDS address 0.
+int grid_kernels_init();
+int launch_grid(int mode, const tsl_filter* f, const Tile& tile, size_t P, size_t N, hipStream_t stream,
+                float* partial, void* trace_out);
+int launch_grid_batch(const BatchLaunch& b, hipStream_t stream, uint32_t* grid_out);
 int batch_grid(const BatchLaunch& b, uint32_t* grid);
 // Automatic chunk length of a batch member with an N-point scan.
 uint32_t batch_chunk(size_t N);
