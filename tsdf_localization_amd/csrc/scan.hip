@@ -399,13 +399,20 @@ static int bucket_scan_temp_bytes(size_t* bytes)
     return TSL_OK;
 }
 
+int particle_order_keys_bytes(size_t n, size_t* bytes)
+{
+    size_t temp = 0;
+    TSL_TRY(bucket_scan_temp_bytes(&temp));
+    *bytes = 2 * round256(sizeof(uint32_t) * kBuckets) + round256(sizeof(uint32_t) * n) + round256(temp);
+    return TSL_OK;
+}
+
 int reserve_particle_order(tsl_filter* f)
 {
     const size_t n = f->count_bound;
-    size_t temp = 0;
-    TSL_TRY(bucket_scan_temp_bytes(&temp));
-    TSL_TRY(f->pkeys.reserve(2 * round256(sizeof(uint32_t) * kBuckets) + round256(sizeof(uint32_t) * n) +
-                             round256(temp)));
+    size_t keys = 0;
+    TSL_TRY(particle_order_keys_bytes(n, &keys));
+    TSL_TRY(f->pkeys.reserve(keys));
     TSL_TRY(f->porder.reserve(sizeof(uint32_t) * n));
     return f->pinv.reserve(sizeof(uint32_t) * n);
 }

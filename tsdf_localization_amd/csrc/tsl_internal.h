@@ -456,6 +456,7 @@ int launch_prep_points(tsl_filter* f, hipStream_t stream);
 size_t prep_points_temp_bytes(uint32_t n);
 // Buffers of the spatial particle order for f->count_bound particles.
 int reserve_particle_order(tsl_filter* f);
+int particle_order_keys_bytes(size_t n, size_t* bytes);  // of f->pkeys for n particles
 // Spatial particle order of a filter and its pose matrices in that order
 // (f->L slot s = particle f->porder[s], f->pinv the inverse), for a filter
 // evaluated as a batch member whose inv points at f->pinv.
