@@ -472,9 +472,8 @@ int tsl_batch_destroy(tsl_batch* b);
 /* Tile of the batched evaluation (k particles per wavefront, 1 or 2; points
  * per lane 1, 2 or 4; chunk_len points per chunk, 0 = automatic: 2048, or
  * the whole scan if shorter).  The workgroups of the persistent grid claim
- * work items (4k particles x one chunk) one at a time; on a map with a class
- * grid its wavefronts do (2 particles x one chunk, whatever k and
- * points_per_lane).  Re-prepares the batch. */
+ * work items (4k particles x one chunk; on a map with a class grid 8, 16 or 32
+ * particles, whatever k and points_per_lane) one at a time.  Re-prepares the batch. */
 int tsl_batch_set_tile(tsl_batch* b, int k, int points_per_lane, uint32_t chunk_len);
 
 /* Time the batched update (every member, reps launches per candidate on

@@ -804,10 +804,10 @@ int dispatch_eval_batch(const BatchLaunch& b, hipStream_t stream, uint32_t* grid
 
 uint32_t batch_item_particles(const tsl_map* map, int K, uint64_t rows)
 {
-    return map->grid.ready ? grid_item_particles(rows) : (uint32_t)(kWaves * K);
+    return map->grid.ready ? grid_item_particles(map->grid, rows) : (uint32_t)(kWaves * K);
 }
 
-uint32_t batch_group_items(const tsl_map* map) { return map->grid.ready ? grid_threads(map->grid) / 64 : 1u; }
+uint32_t batch_group_waves(const tsl_map* map) { return map->grid.ready ? grid_threads(map->grid) / 64 : kWaves; }
 
 int batch_grid(const BatchLaunch& b, uint32_t* grid) { return dispatch_eval_batch(b, nullptr, grid); }
 

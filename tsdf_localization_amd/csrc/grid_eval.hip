@@ -1,8 +1,7 @@
-// Scoring kernels on a map's class grid (class_grid.hip).  A wavefront takes an
-// item of two particles x one chunk of the scan (a few times two where there
-// would be too many items), lane l the points base + l; every lane adds its
-// points in ascending order and the wavefront sums with the same butterfly as
-// eval_kernels.h, so the weights are its bit for bit.
+// Scoring kernels on a map's class grid (class_grid.hip).  A wavefront takes
+// two particles x one chunk of the scan, lane l the points base + l; every
+// lane adds its points in ascending order and the wavefront sums with the same
+// butterfly as eval_kernels.h, so the weights are its bit for bit.
 //
 // Per pair: the exact float transform, one bucket entry per axis (the class
 // boundary and the address terms on its two sides), the sum of the three
@@ -14,18 +13,14 @@
 // recomputed with the reference's arithmetic.
 //
 // 100,000 particles x 20,000 points of the benchmark's building:
-// 3.05 ms against 3.84 (6.5e11 pairs/s against 5.2e11).  What bounds it there
-// is no longer VALU issue (2.2 ms with the gathers taken out) but the cell
-// lines that miss an XCD's L2: 136M of 128 B, 45 G lines/s where random lines
-// reach 56 G.  Two particles are in flight per wavefront because more of them
-// (4, 8) put more distinct cells in flight than the L2 holds (145M, 241M
-// misses), and one leaves the LDS reads' latency bare.
+// 2.54 ms against 3.84 (7.9e11 pairs/s against 5.2e11), close to VALU issue
+// (2.2 ms with the gathers taken out).  The rest is cell lines that miss an
+// XCD's L2.  Two particles are in flight per wavefront because more of them
+// (4, 8) put more distinct cells in flight than the L2 holds.
 //
 // The tables take tens of KB of LDS on large maps, so a workgroup has 4, 8 or
 // 16 wavefronts, whichever keeps most of them resident (grid_threads), and
-// stays: each wavefront goes from item to item on its own, and the points come
-// straight from the L2 one iteration ahead, so that nothing after the staging
-// of the tables makes a wavefront wait for another.
+// stays.  The points come straight from the caches, one iteration ahead.
 #include "eval_kernels.h"
 
 namespace tsl {
@@ -153,19 +148,31 @@ __device__ __forceinline__ void transform(const float (&m)[12], const float4& q,
     tz = m[8] * q.x + m[9] * q.y + m[10] * q.z + m[11];
 }
 
-constexpr int K = (int)grid_item_particles(0);  // particles worked on at a time
+constexpr int K = (int)kGridParticles;
+
+// Points between two barriers of a workgroup's wavefronts.  In step, the 2 x 16
+// neighbouring particles of a workgroup put the same points into the same few
+// metres of the map, so that most of their cells come from lines that another
+// wavefront has just brought in.  100,000 particles x 20,000 points: 3.05 ms
+// without the barriers, 2.59, 2.55, 2.52 ms with one every 128, 256, 512
+// points; 1,000,000 x 3989: 18.5 ms, 12.6, 12.8, 13.0.  (Workgroups of an XCD
+// waiting for each other as well save more lines than the waiting is worth: 11
+// ms there, but 2.7 above.)
+constexpr uint32_t kPace = 256;
 
 // One wavefront: particles p0, p0 + 1 x the points [j0, j1) of one chunk
 // (kMode 0), or the value of every pair to trace_out in the caller's point
-// order (kMode 2).
+// order (kMode 2).  A wavefront with nothing to do (live false) only meets
+// the others at the `paces` barriers.
 template <int kMode, bool kF32>
 __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& g, const ScoreTerm& sc,
                                           const GridTables& tab, const float* __restrict__ L, uint32_t P, uint32_t p0,
-                                          const float4* __restrict__ pts, uint32_t N, uint32_t j0, uint32_t j1,
-                                          float a_hit, float* __restrict__ partial_row, void* __restrict__ trace_out,
-                                          const uint32_t* __restrict__ perm)
+                                          bool live, const float4* __restrict__ pts, uint32_t N, uint32_t j0,
+                                          uint32_t j1, uint32_t paces, float a_hit, float* __restrict__ partial_row,
+                                          void* __restrict__ trace_out, const uint32_t* __restrict__ perm)
 {
     const uint32_t lane = threadIdx.x & 63;
+    if (!live) j1 = j0;
     float m[K][12];
     bool tame = true;
 #pragma unroll
@@ -232,6 +239,7 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
     // its loads take the running offset from a scalar register and read zero
     // past the chunk's end.
     const uint32_t lane_off = lane * 16u;
+    uint32_t met = 0;
     for (uint32_t seg = __builtin_amdgcn_readfirstlane(j0); seg < j1; seg += kSegment) {
         const uint32_t len = min(j1 - seg, kSegment);
         const auto rsrc = point_buffer(pts + seg, len);
@@ -295,6 +303,10 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
         fetch();
         uint32_t off = 0;
         for (; off + 128 <= len; off += 128) {
+            if (off % kPace == 0) {
+                __builtin_amdgcn_s_barrier();
+                ++met;
+            }
             turn(odd, even, off, std::true_type{});
             turn(even, odd, off + 64, std::true_type{});
         }
@@ -303,20 +315,25 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
             odd = even;
         }
     }
+    for (; met < paces; ++met) __builtin_amdgcn_s_barrier();
     if (kMode != 0) return;
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = wave_sum(acc[k]);
-    if (lane == 0) {
+    if (lane == 0 && live) {
 #pragma unroll
         for (int k = 0; k < K; ++k)
             if (p0 + k < P) partial_row[p0 + k] = acc[k];
     }
 }
 
-// Wavefronts of the persistent grid: those of XCD x (workgroups are dealt to
+// Items of a workgroup: `per` particles (kGridParticles for each of its
+// wavefronts; a few times that where there would be too many items) x one
+// chunk, all wavefronts on the same points.  The workgroups of XCD x (dealt to
 // the 8 XCDs round-robin by index) take the items of the x-th contiguous
 // eighth in order, neighbours in the evaluation order together, so that
-// spatially sorted particles share that XCD's L2.
+// spatially sorted particles share that XCD's L2.  (Dealing the last, partial
+// round out by wavefronts instead, a few to every workgroup, measured 2.61 ms
+// against 2.54 at 100,000 x 20,000.)
 template <int kMode, bool kF32>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_eval_grid(
     const DevMap* __restrict__ map_dev, DevGrid g, ScoreTerm sc, const float* __restrict__ L,
@@ -329,23 +346,25 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     const uint32_t xcd = blockIdx.x % kXcds;
     const uint32_t q = items / kXcds, rem = items % kXcds;
     const uint32_t first = xcd * q + min(xcd, rem), end = first + q + (xcd < rem ? 1u : 0u);
-    const uint32_t waves = blockDim.x >> 6;
-    const uint32_t step = gridDim.x / kXcds * waves;  // wavefronts of this XCD (gridDim.x is a multiple of kXcds)
+    const uint32_t waves = blockDim.x >> 6, paces = (chunk_len + kPace - 1) / kPace;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (first + blockIdx.x / kXcds * waves >= end) return;  // uniform across the workgroup
+    uint32_t item = first + blockIdx.x / kXcds;
+    if (item >= end) return;  // uniform across the workgroup
     const GridLds s = stage_grid<kF32>(g, kMode == 0, a_hit);
     const GridTables tab = grid_tables(g, s);
-    for (uint32_t item = first + blockIdx.x / kXcds * waves + wave; item < end; item += step) {
-        const uint32_t grp = item / chunks, c = item - grp * chunks;
-        const uint32_t j0 = c * chunk_len, p1 = min(P, (grp + 1) * per);
-        for (uint32_t p0 = grp * per; p0 < p1; p0 += K)
-            grid_wave<kMode, kF32>(map_dev, g, sc, tab, L, P, p0, pts, N, j0, min(N, j0 + chunk_len), a_hit,
-                                   kMode == 0 ? partial + (size_t)c * stride : nullptr, trace_out, perm);
+    for (; item < end; item += gridDim.x / kXcds) {  // (gridDim.x is a multiple of kXcds)
+        const uint32_t row = item / chunks, c = item - row * chunks;
+        const uint32_t j0 = c * chunk_len;
+        for (uint32_t part = 0; part < per; part += K * waves) {
+            const uint32_t p0 = row * per + part + K * wave;
+            grid_wave<kMode, kF32>(map_dev, g, sc, tab, L, P, p0, p0 < P, pts, N, j0, min(N, j0 + chunk_len), paces,
+                                   a_hit, kMode == 0 ? partial + (size_t)c * stride : nullptr, trace_out, perm);
+        }
     }
 }
 
-// Batched form: every wavefront claims its items one at a time from its XCD's
-// counter (k_eval_batch's claims, without the workgroup's barriers).
+// Batched form: every workgroup claims its items one at a time from its XCD's
+// counter, the next one while it works on an item.
 template <bool kF32>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_eval_grid_batch(
     const DevMap* __restrict__ map_dev, DevGrid g, ScoreTerm sc, const Member* __restrict__ members,
@@ -353,21 +372,20 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
 {
     const GridLds s = stage_grid<kF32>(g, true, a_hit);
     const GridTables tab = grid_tables(g, s);
+    // two claims behind the tables, read and written by turns
+    volatile auto* claimed = reinterpret_cast<volatile __attribute__((address_space(3))) uint32_t*>(
+        (uintptr_t)(grid_lds_bytes(g) - 16));
     const uint32_t n = plan->n;
     const uint32_t total = min(plan->total, item0 + min(count, 0xffffffffu - item0));
     const uint32_t xcd = blockIdx.x % kPlanXcds;
+    const uint32_t waves = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t* counter = &plan->next[xcd * 32];
-    for (;;) {
-        // The wavefront's first lane claims for all.  Its lane number is made
-        // opaque on every turn: a branch that the compiler knows to repeat
-        // lets it give the other lanes a loop of their own around the claim,
-        // in which readfirstlane no longer sees the first lane's (and which
-        // never ends).
-        uint32_t claimer = threadIdx.x & 63u, claim = 0;
-        asm volatile("" : "+v"(claimer));
-        if (claimer == 0) claim = atomicAdd(counter, 1u);
-        const uint32_t item = item0 + __builtin_amdgcn_readfirstlane(claim) * kPlanXcds + xcd;
+    if (threadIdx.x == 0) claimed[0] = atomicAdd(counter, 1u);
+    for (uint32_t turn = 0;; ++turn) {
+        __syncthreads();
+        const uint32_t item = item0 + __builtin_amdgcn_readfirstlane(claimed[turn & 1]) * kPlanXcds + xcd;
         if (item >= total) break;
+        if (threadIdx.x == 0) claimed[(turn + 1) & 1] = atomicAdd(counter, 1u);
         uint32_t lo = 0, hi = n;  // member: prefix[lo] <= item < prefix[lo + 1]
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -376,11 +394,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
         const uint32_t f = __builtin_amdgcn_readfirstlane(lo);
         const Member& mb = members[f];
         const uint32_t local = item - plan->prefix[f];
-        const uint32_t grp = local / mb.chunks, c = local - grp * mb.chunks;
-        const uint32_t j0 = c * mb.chunk_len, P = mb.st->count, p1 = min(P, (grp + 1) * per);
-        for (uint32_t p0 = grp * per; p0 < p1; p0 += K)
-            grid_wave<0, kF32>(map_dev, g, sc, tab, mb.L, P, p0, mb.points, mb.N, j0, min(mb.N, j0 + mb.chunk_len),
-                               a_hit, mb.partial + (size_t)c * mb.stride, nullptr, nullptr);
+        const uint32_t row = local / mb.chunks, c = local - row * mb.chunks;
+        const uint32_t j0 = c * mb.chunk_len, P = mb.st->count, paces = (mb.chunk_len + kPace - 1) / kPace;
+        for (uint32_t part = 0; part < per; part += K * waves) {
+            const uint32_t p0 = row * per + part + K * wave;
+            grid_wave<0, kF32>(map_dev, g, sc, tab, mb.L, P, p0, p0 < P, mb.points, mb.N, j0,
+                               min(mb.N, j0 + mb.chunk_len), paces, a_hit, mb.partial + (size_t)c * mb.stride, nullptr,
+                               nullptr);
+        }
     }
 }
 
@@ -391,11 +412,11 @@ int launch_grid_t(const tsl_filter* f, const Tile& tile, size_t P, size_t N, hip
     constexpr auto kernel = &k_eval_grid<kMode, kF32>;
     const tsl_map* map = f->ev->map;
     const uint32_t threads = grid_threads(map->grid);
-    const uint32_t per = grid_item_particles(P * tile.chunks);
+    const uint32_t per = grid_item_particles(map->grid, P * tile.chunks);
     const size_t items = (P + per - 1) / per * tile.chunks;
     uint32_t groups = 0;
     TSL_TRY(resident_groups(reinterpret_cast<const void*>(kernel), (int)threads, grid_lds_bytes(map->grid),
-                            map->device, (items + threads / 64 - 1) / (threads / 64), &groups));
+                            map->device, items, &groups));
     FilterState* st = f->state.as<FilterState>();
     hipLaunchKernelGGL(kernel, dim3(groups), dim3(threads), grid_lds_bytes(map->grid), stream,
                        map->dev_copy.as<DevMap>(), map->grid, score_term_of(f->ev), f->L.as<float>(), &st->count,
@@ -412,8 +433,8 @@ int launch_grid_batch_t(const BatchLaunch& b, hipStream_t stream, uint32_t* grid
     const uint32_t threads = grid_threads(b.map->grid);
     const size_t lds = grid_lds_bytes(b.map->grid);
     if (grid_out)
-        return resident_groups(reinterpret_cast<const void*>(kernel), (int)threads, lds, b.map->device,
-                               (b.max_items + threads / 64 - 1) / (threads / 64), grid_out);
+        return resident_groups(reinterpret_cast<const void*>(kernel), (int)threads, lds, b.map->device, b.max_items,
+                               grid_out);
     return launch_slices(b, stream, [&](uint32_t item0, uint32_t count) {
         hipLaunchKernelGGL(kernel, dim3(b.grid), dim3(threads), lds, stream, b.map->dev_copy.as<DevMap>(),
                            b.map->grid, b.score, b.members, b.plan, b.a_hit, b.per, item0, count);

@@ -230,8 +230,6 @@ int dispatch(tsl_server* s, Slot* sl)
     const uint32_t n = (uint32_t)sl->reqs.size();
     uint64_t rows = 0;
     uint32_t max_cap = 0;
-    const uint64_t at_once = batch_group_items(s->ev->map);  // items a workgroup works on at a time
-    const uint64_t group_waves = s->ev->map->grid.ready ? at_once : 4;
     // every scan of the tick: one upload, one preparation
     uint32_t total = 0, max_np = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -342,10 +340,10 @@ int dispatch(tsl_server* s, Slot* sl)
     // slice_pairs pairs
     uint64_t grid = (uint64_t)s->per_cu[sl->cls] * (uint64_t)s->cus;
     if (sl->cls == 1 && s->slice_pairs) {
-        const uint64_t keep = (uint64_t)s->reserved_per_cu * 4 * (uint64_t)s->cus / group_waves;
+        const uint64_t keep = (uint64_t)s->reserved_per_cu * 4 * (uint64_t)s->cus / batch_group_waves(s->ev->map);
         grid = std::max<uint64_t>((uint64_t)s->cus, grid - std::min(grid, keep));
     }
-    const uint64_t need = ((max_items + at_once - 1) / at_once + 7) / 8 * 8;
+    const uint64_t need = (max_items + 7) / 8 * 8;
     if (grid > need) grid = need;
     grid = std::max<uint64_t>(8, (grid + 7) / 8 * 8);
     l.grid = (uint32_t)grid;
@@ -354,7 +352,7 @@ int dispatch(tsl_server* s, Slot* sl)
         for (uint32_t i = 0; i < n; ++i)
             pairs_per_item =
                 std::max<uint64_t>(pairs_per_item, (uint64_t)per * sl->members_host[i].chunk_len);
-        l.slice_items = std::max<uint64_t>(grid * at_once, s->slice_pairs / std::max<uint64_t>(pairs_per_item, 1));
+        l.slice_items = std::max<uint64_t>(grid, s->slice_pairs / std::max<uint64_t>(pairs_per_item, 1));
     }
     TSL_TRY(launch_motion_members(l.members, sl->motions.as<tsl_motion>(), n, max_cap, st));
     for (uint32_t i = 0; i < n; ++i) {

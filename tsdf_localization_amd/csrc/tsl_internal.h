@@ -208,19 +208,11 @@ constexpr float kGridMagic = 12582912.0f;  // 1.5 * 2^23, bucket 0
 // Scan points at or past this (or not finite) carry a NaN score term on a map
 // with a class grid: the kernels take their pairs through the exact tiers.
 constexpr float kTamePoint = 65536.0f;
-// LDS bytes of the scoring kernels on a class grid: bitmap, palette, bucket tables.
+// LDS bytes of the scoring kernels on a class grid: bitmap, palette, bucket
+// tables and 16 bytes for the batched form's claims.
 constexpr size_t grid_lds_bytes(const DevGrid& g)
 {
-    return g.bits_bytes + 16 * ((g.palette_size + 3ull) / 4) + 16ull * g.entries;
-}
-// Particles of a wavefront's item on a class grid, for particles x chunks in
-// all: two, which the kernel works on at a time, or as many more as keep the
-// items below 2^31.
-constexpr uint32_t grid_item_particles(uint64_t rows)
-{
-    uint32_t per = 2;
-    while (rows / per >= (1ull << 30)) per *= 2;
-    return per;
+    return g.bits_bytes + 16 * ((g.palette_size + 3ull) / 4) + 16ull * g.entries + 16;
 }
 // Threads of a workgroup: the fewest wavefronts (4, 8 or 16) that keep as many
 // as possible resident on a CU (160 KB of LDS, 32 wavefronts).
@@ -236,6 +228,16 @@ constexpr uint32_t grid_threads(const DevGrid& g)
         }
     }
     return best;
+}
+constexpr uint32_t kGridParticles = 2;  // particles a wavefront works on at a time
+// Particles of a workgroup's item (x one chunk), for particles x chunks in
+// all: kGridParticles a wavefront, or as many times that as keep the items
+// below 2^30.
+constexpr uint32_t grid_item_particles(const DevGrid& g, uint64_t rows)
+{
+    uint32_t per = kGridParticles * (grid_threads(g) / 64);
+    while (rows / per >= (1ull << 30)) per *= 2;
+    return per;
 }
 constexpr size_t kGridLdsBudget = 80 << 10;  // two workgroups of 16 wavefronts on a CU's 160 KB
 
@@ -523,10 +525,10 @@ struct BatchLaunch {
 };
 int launch_batch_update(const BatchLaunch& b, hipStream_t stream);
 // Particles of an item of the batched evaluation (x one chunk) with K particles
-// per wavefront and `rows` particles x chunks over all members, and the items
-// a workgroup works on at a time.
+// per wavefront and `rows` particles x chunks over all members, and the
+// wavefronts of a workgroup of its kernel.
 uint32_t batch_item_particles(const tsl_map* map, int K, uint64_t rows);
-uint32_t batch_group_items(const tsl_map* map);
+uint32_t batch_group_waves(const tsl_map* map);
 // Scoring (mode 0) or value trace (mode 2) on a map's class grid (grid_eval.hip).
 // init, once per map on its device: the kernels may need more dynamic LDS than
 // the runtime grants unasked, and read their tables from LDS address 0.
