@@ -35,7 +35,7 @@ HIP_FLAGS = [
 ]
 
 HIP_SOURCES = ["api.hip", "eval.hip", "resample.hip", "tables.hip", "scan.hip", "batch.hip", "motion.hip", "mcl.hip", "server.hip", "chunks.hip",
-               "class_grid.hip", "grid_eval.hip", "noalloc.hip", "probe.hip"]
+               "class_grid.hip", "grid_eval.hip", "reduce.hip", "noalloc.hip", "probe.hip"]
 # eval_tiles.hip is compiled once per evaluation tile shape (particles per
 # wavefront, points per lane), so that the kernel instantiations build in
 # parallel

@@ -1376,18 +1376,19 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     TSL_TRY(filter_reserve_points(f, n));
     TSL_TRY(f->raw_in.reserve(sizeof(tsl_point) * (n ? n : 1)));
     const size_t ring_room = (ring_bytes * (n ? n : 1) + 3) & ~(size_t)3;
-    TSL_TRY(f->raw_ring.reserve(ring_room + 16));  // rings, then two aligned counters
+    TSL_TRY(f->raw_ring.reserve(ring_room + 16));  // rings, then three aligned counters
     uint32_t* counters = reinterpret_cast<uint32_t*>(f->raw_ring.as<char>() + ring_room);
-    const uint32_t zero[2] = {0u, 0u};
-    TSL_HIP_CHECK(hipMemcpy(counters, zero, sizeof(zero), hipMemcpyHostToDevice));
-    uint32_t host[2] = {0u, 0u};
+    uint32_t host[3] = {0u, 0u, 0u};
     if (n) {
         TSL_HIP_CHECK(hipMemcpy(f->raw_in.ptr, raw, sizeof(tsl_point) * n, hipMemcpyHostToDevice));
         TSL_HIP_CHECK(hipMemcpy(f->raw_ring.ptr, ring, ring_bytes * n, hipMemcpyHostToDevice));
         TSL_TRY(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
-                                   f->points_in.as<tsl_point>(), counters, counters + 1, 0));
+                                   f->points_in.as<tsl_point>(), counters, 0));
         TSL_HIP_CHECK(hipDeviceSynchronize());
         TSL_HIP_CHECK(hipMemcpy(host, counters, sizeof(host), hipMemcpyDeviceToHost));
+        if (host[2])
+            TSL_TRY(launch_reduce_order(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
+                                        f->points_in.as<tsl_point>(), counters, 0));
     }
     if (host[1]) return set_error(TSL_ERR_INVALID_ARGUMENT, "a kept point's ring is outside [0, 64)");
     f->num_points = host[0];

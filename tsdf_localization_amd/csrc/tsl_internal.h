@@ -485,7 +485,9 @@ int filter_reserve_scan(tsl_filter* f, size_t n);
 constexpr int kReduceEvaluator = 0;
 constexpr int kReduceCloud = 1;
 int launch_reduce_scan(tsl_filter* f, int mode, const tsl_point* raw, const void* ring, uint32_t n, float cell,
-                       tsl_point* out, uint32_t* count_dev, uint32_t* bad_dev, hipStream_t stream);
+                       tsl_point* out, uint32_t* counters, hipStream_t stream);
+int launch_reduce_order(tsl_filter* f, int mode, const tsl_point* raw, const void* ring, uint32_t n, float cell,
+                        tsl_point* out, uint32_t* counters, hipStream_t stream);
 
 // Resampling (resample.hip): members[0..n) resampled in one sequence of
 // launches; grid_cap = max cap_limit over the members.
