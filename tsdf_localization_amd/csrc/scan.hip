@@ -51,13 +51,17 @@ __device__ __forceinline__ uint64_t cell_coord(float x)
     return (uint64_t)c;
 }
 
+__device__ __forceinline__ uint64_t morton_key(const tsl_point& p)
+{
+    return spread3(cell_coord(p.x)) | (spread3(cell_coord(p.y)) << 1) | (spread3(cell_coord(p.z)) << 2);
+}
+
 __global__ void k_morton(const tsl_point* __restrict__ in, uint32_t n, uint64_t* __restrict__ keys,
                          uint32_t* __restrict__ vals)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const tsl_point p = in[i];
-    keys[i] = spread3(cell_coord(p.x)) | (spread3(cell_coord(p.y)) << 1) | (spread3(cell_coord(p.z)) << 2);
+    keys[i] = morton_key(in[i]);
     vals[i] = i;
 }
 
@@ -79,6 +83,115 @@ __global__ void k_prep_sorted(const tsl_point* __restrict__ in, const uint32_t* 
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     out[j] = scored_point(in[perm[j]], sc, mark);
+}
+
+// Scans of up to kMergePoints points are sorted in two launches, with the key
+// and the score term formed in them: tiles of 256 points by a bitonic network,
+// then every point's place from its rank in its own tile and a binary search in
+// each of the others (ties in tile order, which is the caller's), staged in LDS
+// 8192 keys at a time.  The time is latency: 9 us of kernels at 701 points, 13
+// at 2056, 18 at 10,000, where key, radix sort and gather kernels took 24, 27
+// and 42 (their merge passes are launches of 5 us each).  The searches grow with
+// the square of the points: a whole call that sets a scan is 44 us against 75 at
+// 10,000 points, 92 against 116 at 65,536, and the two meet near 100,000.
+constexpr uint32_t kSortTile = 256;
+constexpr uint32_t kMergeKeys = 8192;  // 64 KB of LDS
+constexpr uint32_t kMergePoints = 65536;
+
+// One tile per workgroup: its sorted keys (padded to a whole tile) and caller
+// indices.
+__global__ __launch_bounds__(kSortTile) void k_sort_tile(const tsl_point* __restrict__ in, uint32_t n,
+                                                         uint64_t* __restrict__ keys, uint32_t* __restrict__ vals)
+{
+    __shared__ uint64_t other_key[kSortTile];
+    __shared__ uint32_t other_idx[kSortTile];
+    const uint32_t t = threadIdx.x, at = blockIdx.x * kSortTile + t;
+    uint64_t key = at < n ? morton_key(in[at]) : ~0ull;  // (keys have 63 bits: the padding comes last)
+    uint32_t idx = at;
+#pragma unroll
+    for (uint32_t k = 2; k <= kSortTile; k <<= 1) {
+#pragma unroll
+        for (uint32_t j = k >> 1; j; j >>= 1) {
+            uint64_t ok;
+            uint32_t oi;
+            if (j >= 64) {
+                __syncthreads();  // the previous exchange has been read
+                other_key[t] = key;
+                other_idx[t] = idx;
+                __syncthreads();
+                ok = other_key[t ^ j];
+                oi = other_idx[t ^ j];
+            } else {
+                ok = __shfl_xor((unsigned long long)key, (int)j, 64);
+                oi = __shfl_xor(idx, (int)j, 64);
+            }
+            const bool less = key < ok || (key == ok && idx < oi);
+            const bool keep_less = ((t & k) == 0) == ((t & j) == 0);
+            if (less != keep_less) {
+                key = ok;
+                idx = oi;
+            }
+        }
+    }
+    if (at < n || gridDim.x > 1) keys[at] = key;  // (2n keys hold two or more whole tiles)
+    if (at < n) vals[at] = idx;
+}
+
+// A point comes after the keys up to its own in an earlier tile and below its
+// own in a later one.
+constexpr uint32_t kSearches = 8;     // tiles searched at a time
+constexpr uint32_t kMergeGroups = 4;  // groups of threads per tile, each with a share of the searches
+__global__ __launch_bounds__(kSortTile * kMergeGroups) void k_merge_tiles(
+    const tsl_point* __restrict__ in, uint32_t n, ScoreTerm sc, int mark, const uint64_t* __restrict__ keys,
+    const uint32_t* __restrict__ vals, uint32_t* __restrict__ perm, float4* __restrict__ out)
+{
+    __shared__ uint64_t staged[kMergeKeys];
+    const uint32_t t = threadIdx.x % kSortTile, group = threadIdx.x / kSortTile;
+    const uint32_t own = blockIdx.x, tiles = gridDim.x, at = own * kSortTile + t;
+    const uint64_t key = at < n ? keys[at] : ~0ull;
+    const uint32_t idx = at < n ? vals[at] : 0u;
+    const tsl_point p = in[idx];
+    uint32_t before = 0;
+    for (uint32_t t0 = 0; tiles > 1 && t0 < tiles; t0 += kMergeKeys / kSortTile) {
+        const uint32_t here = min(tiles - t0, kMergeKeys / kSortTile);
+        if (t0) __syncthreads();
+        const uint4* src = reinterpret_cast<const uint4*>(keys + t0 * kSortTile);
+        uint4* dst = reinterpret_cast<uint4*>(staged);
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < here * (kSortTile / 2); i += kSortTile * kMergeGroups) dst[i] = src[i];
+        __syncthreads();
+        for (uint32_t s0 = group; s0 < here; s0 += kSearches * kMergeGroups) {
+            uint32_t pos[kSearches];
+            uint64_t bound[kSearches];
+#pragma unroll
+            for (uint32_t q = 0; q < kSearches; ++q) {
+                const uint32_t tile = s0 + q * kMergeGroups;
+                pos[q] = min(tile, here - 1) * kSortTile;
+                bound[q] = key + (t0 + tile < own ? 1u : 0u);
+            }
+#pragma unroll
+            for (uint32_t step = kSortTile / 2; step; step >>= 1) {
+#pragma unroll
+                for (uint32_t q = 0; q < kSearches; ++q) pos[q] += staged[pos[q] + step - 1] < bound[q] ? step : 0u;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kSearches; ++q) {
+                const uint32_t tile = s0 + q * kMergeGroups;
+                pos[q] += staged[pos[q]] < bound[q] ? 1u : 0u;
+                if (tile < here && t0 + tile != own) before += pos[q] - tile * kSortTile;
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t* parts = reinterpret_cast<uint32_t*>(staged);
+    if (group) parts[group * kSortTile + t] = before;
+    __syncthreads();
+    if (group || at >= n) return;
+    uint32_t place = t + before;
+#pragma unroll
+    for (uint32_t g = 1; g < kMergeGroups; ++g) place += parts[g * kSortTile + t];
+    perm[place] = idx;
+    out[place] = scored_point(p, sc, mark);
 }
 
 // Evaluation order of the particles: a counting sort into Morton-ordered
@@ -292,6 +405,18 @@ int launch_prep_points(tsl_filter* f, hipStream_t stream)
     TSL_TRY(f->perm.reserve(sizeof(uint32_t) * n));
     uint64_t* keys = f->sort_keys.as<uint64_t>();
     uint32_t* vals = f->sort_vals.as<uint32_t>();
+    const tsl_evaluator* ev = f->ev;
+    if (n <= kMergePoints) {
+        const uint32_t tiles = (n + kSortTile - 1) / kSortTile;
+        hipLaunchKernelGGL(k_sort_tile, dim3(tiles), dim3(kSortTile), 0, stream, f->points_in.as<tsl_point>(), n, keys,
+                           vals);
+        TSL_HIP_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_merge_tiles, dim3(tiles), dim3(kSortTile * kMergeGroups), 0, stream, f->points_in.as<tsl_point>(), n,
+                           score_term_of(ev), (int)ev->map->grid.ready, keys, vals, f->perm.as<uint32_t>(),
+                           f->points.as<float4>());
+        TSL_HIP_CHECK(hipGetLastError());
+        return TSL_OK;
+    }
     size_t temp = 0;
     TSL_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, temp, keys, keys + n, vals, f->perm.as<uint32_t>(),
                                                      (int)n, 0, 63, stream));
@@ -301,7 +426,6 @@ int launch_prep_points(tsl_filter* f, hipStream_t stream)
     TSL_HIP_CHECK(hipGetLastError());
     TSL_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(f->sort_temp.ptr, temp, keys, keys + n, vals,
                                                      f->perm.as<uint32_t>(), (int)n, 0, 63, stream));
-    const tsl_evaluator* ev = f->ev;
     hipLaunchKernelGGL(k_prep_sorted, dim3(g), dim3(256), 0, stream, f->points_in.as<tsl_point>(),
                        f->perm.as<uint32_t>(), n, score_term_of(ev), (int)ev->map->grid.ready, f->points.as<float4>());
     TSL_HIP_CHECK(hipGetLastError());
