@@ -87,6 +87,38 @@ int filter_reserve_points(tsl_filter* f, size_t n)
 
 static FilterState* host_state(tsl_filter* f) { return static_cast<FilterState*>(f->host_state); }
 
+// Copies of up to kStageBytes in all between two stage_begin go through pinned
+// memory of the filter: the host does not wait for each of them, only once for
+// all at the end of the call (a pageable copy blocks for about 10 us however
+// small it is).  Larger ones are left to the runtime, whose staging costs them
+// little.  stage_begin: no earlier copy is in flight (the device was waited
+// for).
+constexpr size_t kStageBytes = 256 << 10;
+
+static void stage_begin(tsl_filter* f) { f->stage_used = 0; }
+
+// Room for n bytes of staging, or nullptr.
+static char* stage_take(tsl_filter* f, size_t n)
+{
+    if (f->stage_used + n > kStageBytes) return nullptr;
+    if (!f->stage && hipHostMalloc(reinterpret_cast<void**>(&f->stage), kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        f->stage = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    char* p = f->stage + f->stage_used;
+    f->stage_used += (n + 255) / 256 * 256;
+    return p;
+}
+
+static int stage_in(tsl_filter* f, void* dst, const void* src, size_t n, hipStream_t s)
+{
+    char* p = stage_take(f, n);
+    if (p) std::memcpy(p, src, n);
+    TSL_HIP_CHECK(hipMemcpyAsync(dst, p ? p : src, n, hipMemcpyHostToDevice, s));
+    return TSL_OK;
+}
+
 // Device descriptor of the filter, uploaded when any of its buffers or its
 // scan changed since the last upload.
 int filter_member(tsl_filter* f, Member** d_member, uint32_t chunk_len, uint32_t chunks, hipStream_t stream)
@@ -846,6 +878,7 @@ int tsl_filter_destroy(tsl_filter* f)
     (void)hipDeviceSynchronize();
     if (f->host_state) (void)hipHostFree(f->host_state);
     if (f->weights_host) (void)hipHostFree(f->weights_host);
+    if (f->stage) (void)hipHostFree(f->stage);
     if (f->motion_host) (void)hipHostFree(f->motion_host);
     if (f->motion_copied) (void)hipEventDestroy(static_cast<hipEvent_t>(f->motion_copied));
     if (f->ev_start) (void)hipEventDestroy(static_cast<hipEvent_t>(f->ev_start));
@@ -876,11 +909,23 @@ int tsl_filter_get_particles(tsl_filter* f, tsl_particle* p, size_t capacity, si
     if (!f || !n) return set_error(TSL_ERR_INVALID_ARGUMENT, "NULL argument");
     TSL_HIP_CHECK(hipSetDevice(f->device));
     TSL_HIP_CHECK(hipDeviceSynchronize());
-    TSL_HIP_CHECK(hipMemcpy(f->host_state, f->state.ptr, sizeof(FilterState), hipMemcpyDeviceToHost));
+    stage_begin(f);
+    // the particles follow the count without waiting for it, as many as the
+    // host expects
+    const size_t guess = p ? std::min(std::min(f->count_bound, capacity), f->particles.bytes / sizeof(tsl_particle)) : 0;
+    char* stage = guess ? stage_take(f, sizeof(tsl_particle) * guess) : nullptr;
+    TSL_HIP_CHECK(hipMemcpyAsync(f->host_state, f->state.ptr, sizeof(FilterState), hipMemcpyDeviceToHost, 0));
+    if (stage)
+        TSL_HIP_CHECK(hipMemcpyAsync(stage, f->particles.ptr, sizeof(tsl_particle) * guess, hipMemcpyDeviceToHost, 0));
+    TSL_HIP_CHECK(hipStreamSynchronize(0));
     const size_t cnt = host_state(f)->count;
     *n = cnt;
     if (cnt > capacity) return set_error(TSL_ERR_CAPACITY, "filter holds %zu particles", cnt);
-    if (cnt) TSL_HIP_CHECK(hipMemcpy(p, f->particles.ptr, sizeof(tsl_particle) * cnt, hipMemcpyDeviceToHost));
+    const size_t got = stage ? std::min(cnt, guess) : 0;
+    if (got) std::memcpy(p, stage, sizeof(tsl_particle) * got);
+    if (cnt > got)
+        TSL_HIP_CHECK(hipMemcpy(p + got, f->particles.as<tsl_particle>() + got, sizeof(tsl_particle) * (cnt - got),
+                                hipMemcpyDeviceToHost));
     return TSL_OK;
 }
 
@@ -891,11 +936,13 @@ int tsl_filter_set_scan(tsl_filter* f, const tsl_point* pts, size_t n, const flo
     TSL_HIP_CHECK(hipSetDevice(f->device));
     TSL_HIP_CHECK(hipDeviceSynchronize());
     TSL_TRY(filter_reserve_points(f, n));
-    if (n) TSL_HIP_CHECK(hipMemcpy(f->points_in.ptr, pts, sizeof(tsl_point) * n, hipMemcpyHostToDevice));
+    stage_begin(f);
+    if (n) TSL_TRY(stage_in(f, f->points_in.ptr, pts, sizeof(tsl_point) * n, 0));
     f->num_points = n;
     std::memcpy(f->tf, tf, sizeof(float) * 16);
     TSL_TRY(launch_prep_points(f, 0));
     TSL_HIP_CHECK(hipDeviceSynchronize());
+    stage_begin(f);
     return TSL_OK;
 }
 
@@ -1253,16 +1300,19 @@ static int evaluate_filter_scan(tsl_evaluator* ev, tsl_filter* f, tsl_particle* 
             return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
         f->weights_host_cap = P;
     }
+    // (an earlier call on this filter that failed may have left its copies)
+    if (f->stage_used) TSL_HIP_CHECK(hipStreamSynchronize(s));
+    stage_begin(f);
     if (points) {
         TSL_TRY(filter_reserve_points(f, N));
-        TSL_HIP_CHECK(hipMemcpyAsync(f->points_in.ptr, points, sizeof(tsl_point) * N, hipMemcpyHostToDevice, s));
+        TSL_TRY(stage_in(f, f->points_in.ptr, points, sizeof(tsl_point) * N, s));
         f->num_points = N;
         std::memcpy(f->tf, tf, sizeof(float) * 16);
         TSL_TRY(launch_prep_points(f, s));
     }
     f->count_bound = 0;
     TSL_TRY(filter_reserve_particles(f, P));
-    TSL_HIP_CHECK(hipMemcpyAsync(f->particles.ptr, particles, sizeof(tsl_particle) * P, hipMemcpyHostToDevice, s));
+    TSL_TRY(stage_in(f, f->particles.ptr, particles, sizeof(tsl_particle) * P, s));
     f->count_bound = P;
     f->count_known = true;
     TSL_TRY(launch_set_count(f, (uint32_t)P, s));
@@ -1271,6 +1321,7 @@ static int evaluate_filter_scan(tsl_evaluator* ev, tsl_filter* f, tsl_particle* 
     TSL_HIP_CHECK(hipMemcpyAsync(hs, f->state.ptr, sizeof(FilterState), hipMemcpyDeviceToHost, s));
     TSL_HIP_CHECK(hipMemcpyAsync(f->weights_host, f->raw.ptr, sizeof(float) * P, hipMemcpyDeviceToHost, s));
     TSL_HIP_CHECK(hipStreamSynchronize(s));
+    stage_begin(f);
     f->count_bound = hs->count;
     pose_from_stats(hs->stats, out_pose);
     TSL_TRY(status_error(hs->status));
@@ -1380,12 +1431,16 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     uint32_t* counters = reinterpret_cast<uint32_t*>(f->raw_ring.as<char>() + ring_room);
     uint32_t host[3] = {0u, 0u, 0u};
     if (n) {
-        TSL_HIP_CHECK(hipMemcpy(f->raw_in.ptr, raw, sizeof(tsl_point) * n, hipMemcpyHostToDevice));
-        TSL_HIP_CHECK(hipMemcpy(f->raw_ring.ptr, ring, ring_bytes * n, hipMemcpyHostToDevice));
+        stage_begin(f);
+        char* result = stage_take(f, sizeof(host));
+        if (!result) return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
+        TSL_TRY(stage_in(f, f->raw_in.ptr, raw, sizeof(tsl_point) * n, 0));
+        TSL_TRY(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0));
         TSL_TRY(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
                                    f->points_in.as<tsl_point>(), counters, 0));
-        TSL_HIP_CHECK(hipDeviceSynchronize());
-        TSL_HIP_CHECK(hipMemcpy(host, counters, sizeof(host), hipMemcpyDeviceToHost));
+        TSL_HIP_CHECK(hipMemcpyAsync(result, counters, sizeof(host), hipMemcpyDeviceToHost, 0));
+        TSL_HIP_CHECK(hipStreamSynchronize(0));
+        std::memcpy(host, result, sizeof(host));
         if (host[2])
             TSL_TRY(launch_reduce_order(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
                                         f->points_in.as<tsl_point>(), counters, 0));
@@ -1395,6 +1450,7 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     std::memcpy(f->tf, tf, sizeof(float) * 16);
     TSL_TRY(launch_prep_points(f, 0));
     TSL_HIP_CHECK(hipDeviceSynchronize());
+    stage_begin(f);
     return TSL_OK;
 }
 
@@ -1446,41 +1502,47 @@ int tsl_resample_systematic(const tsl_particle* in, size_t M, float u0, tsl_part
     size_t cap = 0;
     TSL_TRY(resample_capacity(M, u0, &cap));
     if (cap > 0xffffffffull) return set_error(TSL_ERR_UNSUPPORTED, "resampling output too large");
-    DevBuf d_in, d_out, d_s, d_u, d_idx, d_st, d_plan, d_mem;
-    TSL_TRY(d_in.reserve(sizeof(tsl_particle) * M));
-    TSL_TRY(d_out.reserve(sizeof(tsl_particle) * cap));
-    TSL_TRY(d_s.reserve(sizeof(double) * M));
-    TSL_TRY(d_u.reserve(sizeof(float) * cap));
-    TSL_TRY(d_idx.reserve(sizeof(int32_t) * cap));
-    TSL_TRY(d_st.reserve(sizeof(FilterState)));
-    TSL_TRY(d_plan.reserve(sizeof(RsPlan)));
-    TSL_TRY(d_mem.reserve(sizeof(Member)));
-    TSL_HIP_CHECK(hipMemcpy(d_in.ptr, in, sizeof(tsl_particle) * M, hipMemcpyHostToDevice));
-    FilterState hs{};
-    hs.count = (uint32_t)M;
-    hs.first_bad = 0xffffffffu;
-    TSL_HIP_CHECK(hipMemcpy(d_st.ptr, &hs, sizeof(hs), hipMemcpyHostToDevice));
-    Member h;
-    std::memset(&h, 0, sizeof(h));
-    h.particles = d_in.as<tsl_particle>();
-    h.alt = d_out.as<tsl_particle>();
-    h.st = d_st.as<FilterState>();
-    h.cumsum = d_s.as<double>();
-    h.ubuf = d_u.as<float>();
-    h.idx_out = d_idx.as<int32_t>();
-    h.plan = d_plan.as<RsPlan>();
-    h.cap_limit = (uint32_t)cap;
-    TSL_HIP_CHECK(hipMemcpy(d_mem.ptr, &h, sizeof(h), hipMemcpyHostToDevice));
-    TSL_TRY(launch_resample_members(d_mem.as<Member>(), 1, (uint32_t)cap, u0, false, 0));
-    TSL_HIP_CHECK(hipDeviceSynchronize());
-    TSL_HIP_CHECK(hipMemcpy(&hs, d_st.ptr, sizeof(hs), hipMemcpyDeviceToHost));
+    // one allocation for all the buffers; the state and the descriptor, next to
+    // each other at its head, go up in one copy
+    struct Head {
+        alignas(256) FilterState st;
+        alignas(256) Member mem;
+    } head{};
+    const size_t sizes[] = {sizeof(Head),          sizeof(RsPlan),          sizeof(tsl_particle) * M,
+                            sizeof(tsl_particle) * cap, sizeof(double) * M, sizeof(float) * cap, sizeof(int32_t) * cap};
+    constexpr int kBufs = sizeof(sizes) / sizeof(sizes[0]);
+    size_t at[kBufs], total = 0;
+    for (int k = 0; k < kBufs; ++k) {
+        at[k] = total;
+        total += (sizes[k] + 255) / 256 * 256;
+    }
+    DevBuf buf;
+    TSL_TRY(buf.reserve(total));
+    char* base = buf.as<char>();
+    tsl_particle* d_out = reinterpret_cast<tsl_particle*>(base + at[3]);
+    int32_t* d_idx = reinterpret_cast<int32_t*>(base + at[6]);
+    head.st.count = (uint32_t)M;
+    head.st.first_bad = 0xffffffffu;
+    head.mem.particles = reinterpret_cast<tsl_particle*>(base + at[2]);
+    head.mem.alt = d_out;
+    head.mem.st = reinterpret_cast<FilterState*>(base);
+    head.mem.cumsum = reinterpret_cast<double*>(base + at[4]);
+    head.mem.ubuf = reinterpret_cast<float*>(base + at[5]);
+    head.mem.idx_out = d_idx;
+    head.mem.plan = reinterpret_cast<RsPlan*>(base + at[1]);
+    head.mem.cap_limit = (uint32_t)cap;
+    TSL_HIP_CHECK(hipMemcpy(head.mem.particles, in, sizeof(tsl_particle) * M, hipMemcpyHostToDevice));
+    TSL_HIP_CHECK(hipMemcpy(base, &head, sizeof(head), hipMemcpyHostToDevice));
+    TSL_TRY(launch_resample_members(&reinterpret_cast<Head*>(base)->mem, 1, (uint32_t)cap, u0, false, 0));
+    FilterState& hs = head.st;
+    TSL_HIP_CHECK(hipMemcpy(&hs, base, sizeof(hs), hipMemcpyDeviceToHost));
     if (hs.status == kStCapacity) return set_error(TSL_ERR_CAPACITY, "weights sum beyond 1 + 1e-5: normalise them first");
     if (hs.status != kStOk) return set_error(TSL_ERR_UNSUPPORTED, "resampling failed (status %u)", hs.status);
     const uint32_t J = hs.resample_count;
     *out_count = J;
     if (J > out_capacity) return set_error(TSL_ERR_CAPACITY, "resampling emits %u particles", J);
-    if (out && J) TSL_HIP_CHECK(hipMemcpy(out, d_out.ptr, sizeof(tsl_particle) * J, hipMemcpyDeviceToHost));
-    if (out_indices && J) TSL_HIP_CHECK(hipMemcpy(out_indices, d_idx.ptr, sizeof(int32_t) * J, hipMemcpyDeviceToHost));
+    if (out && J) TSL_HIP_CHECK(hipMemcpy(out, d_out, sizeof(tsl_particle) * J, hipMemcpyDeviceToHost));
+    if (out_indices && J) TSL_HIP_CHECK(hipMemcpy(out_indices, d_idx, sizeof(int32_t) * J, hipMemcpyDeviceToHost));
     return TSL_OK;
 }
 

@@ -426,6 +426,8 @@ struct tsl_filter {
     void* host_state = nullptr;  // pinned FilterState mirror
     void* weights_host = nullptr;  // pinned read-back of the normalised weights (drop-in evaluation)
     size_t weights_host_cap = 0;   // floats it holds
+    char* stage = nullptr;         // pinned staging of small copies (kStageBytes), made on first use
+    size_t stage_used = 0;         // bytes that copies in flight may still read or write
 };
 
 namespace tsl {

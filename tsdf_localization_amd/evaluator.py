@@ -279,6 +279,12 @@ def check_invtrig_libm(stride, atan2_samples):
     return bad.value, n.value
 
 
+def _head(a, n):
+    """The first n rows of an array nothing else refers to, cut to size in place."""
+    a.resize((n,) + a.shape[1:], refcheck=False)
+    return a
+
+
 def resample_systematic(particles, u0):
     """Device systematic resampling; returns (new_particles, source_indices)."""
     p = _particles(particles)
@@ -289,7 +295,7 @@ def resample_systematic(particles, u0):
     idx = np.empty(max(cap.value, 1), np.int32)
     n = ctypes.c_size_t()
     check(lib.tsl_resample_systematic(ptr(p), M, float(u0), ptr(out), out.shape[0], ptr(idx), ctypes.byref(n)))
-    return out[: n.value].copy(), idx[: n.value].copy()
+    return _head(out, n.value), _head(idx, n.value)
 
 
 class ParticleCloud:
@@ -386,7 +392,7 @@ class DeviceFilter:
             capacity = n.value
         out = np.empty((max(capacity, 1), 7), np.float32)
         check(lib.tsl_filter_get_particles(self.handle, ptr(out), capacity, ctypes.byref(n)))
-        return out[: n.value].copy()
+        return _head(out, n.value)
 
     def set_scan(self, points, tf_matrix):
         pts = _points(points)
@@ -419,7 +425,7 @@ class DeviceFilter:
         lib.tsl_filter_get_scan(self.handle, None, 0, ctypes.byref(n))
         out = np.empty((max(n.value, 1), 3), np.float32)
         check(lib.tsl_filter_get_scan(self.handle, ptr(out), out.shape[0], ctypes.byref(n)))
-        return out[: n.value].copy()
+        return _head(out, n.value)
 
     def update_async(self, stream=None):
         check(lib.tsl_filter_update_async(self.handle, None if stream is None else stream.handle))
