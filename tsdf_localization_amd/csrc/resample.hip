@@ -34,7 +34,11 @@ namespace tsl {
 namespace {
 
 constexpr int kRsThreads = 1024;
-constexpr uint32_t kRsSmall = 2048;  // a lone filter with at most this many candidates resamples in one launch
+// A lone filter with at most this many candidates resamples in one launch (its
+// running sum, U and weights in 128 KB of LDS).  5,000 particles: 32 us against
+// 43 in seven launches and the gaps between them.  A third of it is thread 0
+// walking the runs of U; past 8192 the LDS is too small.
+constexpr uint32_t kRsSmall = 8192;
 
 __host__ __device__ __forceinline__ float rec_step(float u, double inv_m) { return (float)((double)u + inv_m); }
 
@@ -407,15 +411,17 @@ __global__ void k_rs_copy_back(const Member* __restrict__ members)
 // sequential recurrences and every output is the same; the particles move
 // through registers instead of the alternate buffer when they replace the
 // resident set.
-constexpr int kRsSmallPer = (int)(kRsSmall / kRsThreads);  // particles and candidates per thread
-static_assert(kRsSmall % kRsThreads == 0, "");
+template <int kPer>  // particles and candidates per thread
+constexpr size_t kRsSmallLds = (size_t)kPer * kRsThreads * (sizeof(double) + 2 * sizeof(float));
 
+template <int kPer>
 __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ members, float u0_arg, int copy_back)
 {
+    constexpr uint32_t kMost = (uint32_t)kPer * kRsThreads;
+    extern __shared__ double s_sh[];                       // kMost running sums,
+    float* w_sh = reinterpret_cast<float*>(s_sh + kMost);  // weights
+    float* u_sh = w_sh + kMost;                            // and U
     __shared__ USeg seg_sh[kMaxSeg];
-    __shared__ double s_sh[kRsSmall];
-    __shared__ float w_sh[kRsSmall];
-    __shared__ float u_sh[kRsSmall];
     __shared__ double wave_tot[kRsThreads / 64];
     __shared__ uint32_t count_sh[kRsThreads / 64];
     __shared__ uint32_t s_bad_sh, u_bad_sh, go_sh, cap_sh, nseg_sh;
@@ -427,18 +433,18 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ me
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the weights are read while thread 0 plans the draw
     const uint32_t M = st->count;
-    float w[2];
+    float w[kPer];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint32_t m = 2 * tid + e;
-        w[e] = (m < M && M <= kRsSmall) ? mb.particles[m].second : 0.0f;
+    for (int e = 0; e < kPer; ++e) {
+        const uint32_t m = kPer * tid + e;
+        w[e] = (m < M && M <= kMost) ? mb.particles[m].second : 0.0f;
     }
     if (tid == 0) {
         s_bad_sh = 0xffffffffu;
         u_bad_sh = 0xffffffffu;
         plan_member(mb, u0_arg, seg_sh);
         uint32_t go = p->cap != 0;
-        if (go && (M > kRsSmall || p->cap > kRsSmall)) {  // the launcher keeps both within kRsSmall
+        if (go && (M > kMost || p->cap > kMost)) {  // the launcher keeps both within kMost
             st->status = kStCapacity;
             p->cap = 0;
             go = 0;
@@ -456,18 +462,22 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ me
     const float u0 = u0_sh;
     // running-sum candidates (one span, as k_rs_scan), checked against
     // s_m == s_{m-1} + w_m
-    const double d0 = (double)w[0], d1 = (double)w[1];
-    const double run = d0 + d1;
+    double loc[kPer];
+    double run = 0.0;
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        run += (double)w[e];
+        loc[e] = run;
+        w_sh[kPer * tid + e] = w[e];
+    }
     const double incl = wave_incl_scan(run, (int)lane);
     if (lane == 63) wave_tot[wave] = incl;
-    w_sh[2 * tid] = w[0];
-    w_sh[2 * tid + 1] = w[1];
     __syncthreads();
     double woff = 0.0;
     for (uint32_t k = 0; k < wave; ++k) woff += wave_tot[k];
     const double excl = woff + (incl - run);
-    s_sh[2 * tid] = excl + d0;
-    s_sh[2 * tid + 1] = excl + run;
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) s_sh[kPer * tid + e] = excl + loc[e];
     // U candidates from the run table, checked against one step of the
     // recurrence
     for (uint32_t j = tid; j < cap; j += kRsThreads) {
@@ -478,8 +488,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ me
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint32_t m = 2 * tid + e;
+    for (int e = 0; e < kPer; ++e) {
+        const uint32_t m = tid + (uint32_t)e * kRsThreads;
         if (m < M) {
             const double prev = m == 0 ? 0.0 : s_sh[m - 1];
             if (s_sh[m] != prev + (double)w_sh[m]) atomicMin(&s_bad_sh, m);
@@ -528,9 +538,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ me
     for (int k = 0; k < kRsThreads / 64; ++k) J += count_sh[k];
     // output j is particle min{m : s_m > U_j}, held in registers (its
     // seven floats)
-    float out[kRsSmallPer][7];
+    float out[kPer][7];
 #pragma unroll
-    for (int r = 0; r < kRsSmallPer; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         const uint32_t j = tid + (uint32_t)r * kRsThreads;
 #pragma unroll
         for (int k = 0; k < 7; ++k) out[r][k] = 0.0f;
@@ -558,7 +568,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_small(Member* __restrict__ me
     if (!copy_back) return;
     __syncthreads();  // every source particle is read
 #pragma unroll
-    for (int r = 0; r < kRsSmallPer; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         const uint32_t j = tid + (uint32_t)r * kRsThreads;
         if (j < J) {
 #pragma unroll
@@ -588,7 +598,17 @@ int launch_resample_members(Member* d_members, uint32_t n, uint32_t grid_cap, fl
 {
     if (n == 0) return TSL_OK;
     if (n == 1 && grid_cap <= kRsSmall) {
-        hipLaunchKernelGGL(k_rs_small, dim3(1, 1), dim3(kRsThreads), 0, stream, d_members, u0_arg, copy_back ? 1 : 0);
+        if (grid_cap <= 2 * kRsThreads) {
+            hipLaunchKernelGGL(k_rs_small<2>, dim3(1, 1), dim3(kRsThreads), kRsSmallLds<2>, stream, d_members, u0_arg,
+                               copy_back ? 1 : 0);
+        } else {
+            // (more LDS than the runtime grants unasked; a host call, cheap and
+            // allowed during a capture)
+            TSL_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rs_small<8>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsSmallLds<8>));
+            hipLaunchKernelGGL(k_rs_small<8>, dim3(1, 1), dim3(kRsThreads), kRsSmallLds<8>, stream, d_members, u0_arg,
+                               copy_back ? 1 : 0);
+        }
         TSL_HIP_CHECK(hipGetLastError());
         return TSL_OK;
     }
