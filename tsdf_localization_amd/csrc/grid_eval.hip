@@ -13,9 +13,11 @@
 // recomputed with the reference's arithmetic.
 //
 // 100,000 particles x 20,000 points of the benchmark's building:
-// 2.54 ms against 3.84 (7.9e11 pairs/s against 5.2e11), close to VALU issue
-// (2.2 ms with the gathers taken out).  The rest is cell lines that miss an
-// XCD's L2.  Two particles are in flight per wavefront because more of them
+// 2.57 ms against 3.84 (7.8e11 pairs/s against 5.2e11); VALU instructions issue
+// on 95 % of the cycles (2.2 ms with the gathers taken out).  Where two thirds
+// of the pairs read a cell (tracking filters) the texture-data path is full
+// instead, and a million sparse particles wait for lines beyond the L2.  Two
+// particles are in flight per wavefront because more of them
 // (4, 8) put more distinct cells in flight than the L2 holds.
 //
 // The tables take tens of KB of LDS on large maps, so a workgroup has 4, 8 or
