@@ -473,28 +473,28 @@ TSL_HD double motion_normal(uint64_t seed, uint64_t particle, uint32_t draw)
 // rotated into the particle's frame (translation added, rotation composed)
 // and the new angles are read back as getAngleFromMat does
 // (src/util/util.cpp:86-111).  Float arithmetic left to right, no FMA.
-TSL_HD void apply_motion(const float last[6], const double d[6], float out[6], int trig = kTrigGlibcFma)
+// compose_motion: the same from the float translation and sines and cosines of
+// the step (sd, cd: roll, pitch, yaw) and of the particle's angles (sl, cl).
+TSL_HD void compose_motion(const float last[6], const float dxyz[3], const float sd[3], const float cd[3],
+                           const float sl[3], const float cl[3], float out[6], int trig)
 {
-    const float sin_roll = (float)sin(d[3]), cos_roll = (float)cos(d[3]);
-    const float sin_pitch = (float)sin(d[4]), cos_pitch = (float)cos(d[4]);
-    const float sin_yaw = (float)sin(d[5]), cos_yaw = (float)cos(d[5]);
+    const float sin_roll = sd[0], cos_roll = cd[0];
+    const float sin_pitch = sd[1], cos_pitch = cd[1];
+    const float sin_yaw = sd[2], cos_yaw = cd[2];
     float o[12];
     o[0] = cos_pitch * cos_yaw;
     o[4] = cos_pitch * sin_yaw;
     o[8] = -sin_pitch;
-    o[3] = (float)d[0];
+    o[3] = dxyz[0];
     o[1] = sin_roll * sin_pitch * cos_yaw - cos_roll * sin_yaw;
     o[5] = sin_roll * sin_pitch * sin_yaw + cos_roll * cos_yaw;
     o[9] = sin_roll * cos_pitch;
-    o[7] = (float)d[1];
+    o[7] = dxyz[1];
     o[2] = cos_roll * sin_pitch * cos_yaw + sin_roll * sin_yaw;
     o[6] = cos_roll * sin_pitch * sin_yaw - sin_roll * cos_yaw;
     o[10] = cos_roll * cos_pitch;
-    o[11] = (float)d[2];
-    float sa, ca, sb, cb, sg, cg;
-    sincosf_mode(trig, last[3], &sa, &ca);
-    sincosf_mode(trig, last[4], &sb, &cb);
-    sincosf_mode(trig, last[5], &sg, &cg);
+    o[11] = dxyz[2];
+    const float sa = sl[0], ca = cl[0], sb = sl[1], cb = cl[1], sg = sl[2], cg = cl[2];
     float p[12];
     p[0] = cb * cg;
     p[4] = cb * sg;
@@ -549,6 +549,18 @@ TSL_HD void apply_motion(const float last[6], const double d[6], float out[6], i
     out[3] = roll;
     out[4] = pitch;
     out[5] = yaw;
+}
+
+TSL_HD void apply_motion(const float last[6], const double d[6], float out[6], int trig = kTrigGlibcFma)
+{
+    float dxyz[3], sd[3], cd[3], sl[3], cl[3];
+    for (int k = 0; k < 3; ++k) {
+        dxyz[k] = (float)d[k];
+        sd[k] = (float)sin(d[3 + k]);
+        cd[k] = (float)cos(d[3 + k]);
+        sincosf_mode(trig, last[3 + k], &sl[k], &cl[k]);
+    }
+    compose_motion(last, dxyz, sd, cd, sl, cl, out, trig);
 }
 
 }  // namespace tsl
