@@ -376,9 +376,7 @@ __global__ void k_grid_bits(const uint8_t* __restrict__ flags, uint64_t bricks, 
     bits[b] = (uint8_t)v;
 }
 
-}  // namespace
-
-int build_class_grid(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
+int build(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
 {
     const tsl_map_coef& c = m->coef;
     DevMap& d = m->dev;
@@ -477,6 +475,20 @@ int build_class_grid(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
     g.init = d.init;
     g.ready = 1;
     return grid_kernels_init();
+}
+
+}  // namespace
+
+int build_class_grid(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
+{
+    const int rc = build(m, grid_occ, init_code);
+    if (rc != TSL_ERR_OUT_OF_MEMORY) return rc;
+    // no room beside the map: it is scored without
+    (void)hipGetLastError();
+    clear_error();
+    m->grid = DevGrid{};
+    for (DevBuf* b : {&m->grid_axis, &m->grid_bits, &m->grid_cells, &m->grid_palette}) b->release();
+    return TSL_OK;
 }
 
 }  // namespace tsl
