@@ -111,6 +111,14 @@ static char* stage_take(tsl_filter* f, size_t n)
     return p;
 }
 
+// A call that ends early waits for the copies it has queued: they may still
+// read the caller's arrays.
+static int wait_on_error(int rc)
+{
+    if (rc != TSL_OK) (void)hipDeviceSynchronize();
+    return rc;
+}
+
 static int stage_in(tsl_filter* f, void* dst, const void* src, size_t n, hipStream_t s)
 {
     char* p = stage_take(f, n);
@@ -940,7 +948,7 @@ int tsl_filter_set_scan(tsl_filter* f, const tsl_point* pts, size_t n, const flo
     if (n) TSL_TRY(stage_in(f, f->points_in.ptr, pts, sizeof(tsl_point) * n, 0));
     f->num_points = n;
     std::memcpy(f->tf, tf, sizeof(float) * 16);
-    TSL_TRY(launch_prep_points(f, 0));
+    TSL_TRY(wait_on_error(launch_prep_points(f, 0)));
     TSL_HIP_CHECK(hipDeviceSynchronize());
     stage_begin(f);
     return TSL_OK;
@@ -1435,9 +1443,9 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
         char* result = stage_take(f, sizeof(host));
         if (!result) return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
         TSL_TRY(stage_in(f, f->raw_in.ptr, raw, sizeof(tsl_point) * n, 0));
-        TSL_TRY(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0));
-        TSL_TRY(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
-                                   f->points_in.as<tsl_point>(), counters, 0));
+        TSL_TRY(wait_on_error(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0)));
+        TSL_TRY(wait_on_error(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
+                                                 f->points_in.as<tsl_point>(), counters, 0)));
         TSL_HIP_CHECK(hipMemcpyAsync(result, counters, sizeof(host), hipMemcpyDeviceToHost, 0));
         TSL_HIP_CHECK(hipStreamSynchronize(0));
         std::memcpy(host, result, sizeof(host));
@@ -1448,7 +1456,7 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     if (host[1]) return set_error(TSL_ERR_INVALID_ARGUMENT, "a kept point's ring is outside [0, 64)");
     f->num_points = host[0];
     std::memcpy(f->tf, tf, sizeof(float) * 16);
-    TSL_TRY(launch_prep_points(f, 0));
+    TSL_TRY(wait_on_error(launch_prep_points(f, 0)));
     TSL_HIP_CHECK(hipDeviceSynchronize());
     stage_begin(f);
     return TSL_OK;
