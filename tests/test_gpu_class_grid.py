@@ -51,3 +51,23 @@ def test_class_grid_values_and_weights(name, form):
     q[30, 1] = np.nan
     got = ev.trace_values(parts, q, tf)
     assert np.array_equal(got.view(np.uint32), oracle_values(om, om.trace(parts, q, tf)).view(np.uint32))
+
+
+@pytest.mark.parametrize("N", [131072, 131009])
+def test_scan_ending_on_an_allocation_boundary(N):
+    """131072 points of 16 bytes fill 2 MiB: nothing lies behind the last one
+    for the loads ahead of a chunk's end.  Tolerance: 4 additions to a lane's
+    sum, 6 of the butterfly, 512 chunks of 256 points, 2 in a pair's term."""
+    import tsdf_localization_amd as tsl
+    c, grid, rng = _case("even")
+    c.init_value = 0.0126
+    data = rng.uniform(0.01, 1.0, 300).astype(np.float32)
+    data = np.resize(data, int(c.data_size))
+    ev = tsl.TSDFEvaluator(tsl.CudaSubVoxelMap(c, grid, data=data))
+    parts = np.zeros((5, 7), np.float32)
+    parts[:, :3] = rng.uniform(1.0, 2.0, (5, 3))
+    parts[:, 6] = 0.2
+    pts = rng.uniform(-3.0, 3.0, (N, 3)).astype(np.float32)
+    tf = np.ascontiguousarray(np.eye(4, dtype=np.float32).reshape(-1))
+    _, w64 = ob.OracleMap(c, grid, data).evaluate(parts, pts, tf)
+    assert np.max(rel_err(ev.evaluate_raw(parts, pts, tf), w64)) <= 524 * 2.0 ** -24

@@ -110,9 +110,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t point_buffer(const float4* p, 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float4*>(p), 0, (int)(n * 16u), 0x00020000);
 }
 
-__device__ __forceinline__ float4 point_at(__amdgpu_buffer_rsrc_t rsrc, uint32_t lane_off, uint32_t off)
+// The whole offset goes into the vector operand: a raw buffer's range check
+// covers that and the instruction's constant, not a scalar offset, so a load
+// past the descriptor's end gives zero and reads nothing.
+__device__ __forceinline__ float4 point_at(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte)
 {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)lane_off, (int)off, 0);
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)byte, 0, 0);
     return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
 }
 
@@ -237,9 +240,8 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
             }
         }
     };
-    // The points come through a buffer descriptor of at most kSegment of them:
-    // its loads take the running offset from a scalar register and read zero
-    // past the chunk's end.
+    // The points come through a buffer descriptor of at most kSegment of them,
+    // whose loads give zero past the chunk's end.
     const uint32_t lane_off = lane * 16u;
     uint32_t met = 0;
     for (uint32_t seg = __builtin_amdgcn_readfirstlane(j0); seg < j1; seg += kSegment) {
@@ -263,7 +265,7 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
             // lanes of the exact tiers and marked points (a NaN value of the
             // map or score term is formed again, with the same result)
             if (__builtin_expect((__builtin_amdgcn_ballot_w64(nan) | wild) != 0, 0)) {
-                const float4 q = point_at(rsrc, lane_off, off * 16u);
+                const float4 q = point_at(rsrc, lane_off + off * 16u);
 #pragma unroll
                 for (int k = 0; k < K; ++k)
                     if (wild || sum[k] != sum[k]) {
@@ -291,14 +293,14 @@ __device__ __forceinline__ void grid_wave(const DevMap* map_dev, const DevGrid& 
         // cover loads that some lanes may not have issued.
         auto arrive = [](float4& q) { asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.w)); };
         auto turn = [&](const float4& now, float4& after, uint32_t off, auto full_tag) {
-            after = point_at(rsrc, lane_off, (off + 128u) * 16u);
+            after = point_at(rsrc, lane_off + (off + 128u) * 16u);
             locate(now);
             finish(off, full_tag);
             w = now.w;
             arrive(after);
             fetch();
         };
-        float4 even = point_at(rsrc, lane_off, 0), odd = point_at(rsrc, lane_off, 64u * 16u);
+        float4 even = point_at(rsrc, lane_off), odd = point_at(rsrc, lane_off + 64u * 16u);
         locate(even);
         w = even.w;
         arrive(odd);
