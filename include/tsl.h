@@ -163,11 +163,10 @@ int tsl_map_chunks_to_cells(const int32_t* chunk_pos, const uint32_t* chunk_raw,
 float tsl_likelihood_value(int16_t tsdf_mm, float sigma);
 float tsl_likelihood_init(float sigma);
 
-/* Device bytes of the map as it was loaded: voxels and lookup tables.  A map
- * that is scored through a class grid (the dense copy of its allocated blocks'
+/* Device bytes held by the map: voxels, lookup tables and, where the map is
+ * scored through one, its class grid (the dense copy of its allocated blocks'
  * neighbourhood that the scoring kernels read; at most 4 x data_size + 32M
- * cells of 2 or 4 bytes, below 4 GB) holds that in addition; like a server's
- * tick buffers it is not charged to a server's budget. */
+ * cells of 2 or 4 bytes, below 4 GB).  A server's budget starts from them. */
 int tsl_map_device_bytes(const tsl_map* map, uint64_t* bytes);
 
 int tsl_map_destroy(tsl_map* map);

@@ -1,0 +1,63 @@
+"""Host paths of the library that need a device to run, on the CPU: libtsl.so
+over the stand-in of the HIP runtime in cpp/hip_stub.cpp (device memory is host
+memory, kernels do nothing, asynchronous copies run when something waits for
+them).  Each test runs in a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before libtsl.so
+stub.stub_live_bytes.restype = ctypes.c_size_t
+stub.stub_set_total.argtypes = [ctypes.c_size_t]
+stub.stub_fail_launch.argtypes = [ctypes.c_long]
+import numpy as np
+import tsdf_localization_amd as tsl
+
+def host_map(ext=(3.0, 3.0, 2.0), res=0.05):
+    c = tsl.coef_init((0, 0, 0), ext, res, 0.25)
+    n = int(c.grid_occ_size)
+    sd3 = int(c.sub_dim) ** 3
+    c.data_size = n * sd3
+    grid = (np.arange(n) * sd3).astype(np.int32)
+    return tsl.CudaSubVoxelMap(c, grid, data=np.resize(np.float32([0.5, 0.75]), n * sd3))
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = tmp_path_factory.mktemp("stub") / "libhipstub.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", "/opt/rocm/include", "-o", str(out),
+                    os.path.join(HERE, "cpp", "hip_stub.cpp")], check=True)
+    return out
+
+
+def run(stub, code):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, str(stub)], cwd=os.path.dirname(HERE),
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+@pytest.mark.parametrize("ext,res", [((3.0, 3.0, 2.0), 0.05), ((3.0, 3.0, 2.0), 0.04)])
+def test_map_bytes_and_server_budget_hold_the_class_grid(stub, ext, res):
+    """tsl_map_device_bytes is what the map holds on the device, with a class
+    grid (0.05 m) and without (0.04 m), and a server's budget starts from it."""
+    out = run(stub, f"""
+from tsdf_localization_amd.server import Server
+m = host_map({ext}, {res})
+before = stub.stub_live_bytes()
+d = m.device_map()
+held = stub.stub_live_bytes() - before
+print("voxels", 2 * m.dataSize(), "held", held)
+assert d.device_bytes() == held, (d.device_bytes(), held)
+s = Server(tsl.TSDFEvaluator(m), max_robots=2, max_particles=100)
+assert s.stats()["used_bytes"] == held
+s.close()
+""")
+    print(out)

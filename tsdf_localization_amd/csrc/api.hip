@@ -837,7 +837,8 @@ int tsl_map_device_bytes(const tsl_map* m, uint64_t* bytes)
 {
     if (!m || !bytes) return set_error(TSL_ERR_INVALID_ARGUMENT, "NULL argument");
     *bytes = m->grid_occ.bytes + m->codes.bytes + m->palette.bytes + m->sub_tab.bytes + m->full.bytes +
-             m->neg_tab.bytes + m->occ_words.bytes + m->axis_tab.bytes + m->slots.bytes;
+             m->neg_tab.bytes + m->occ_words.bytes + m->axis_tab.bytes + m->slots.bytes + m->grid_axis.bytes +
+             m->grid_bits.bytes + m->grid_cells.bytes + m->grid_palette.bytes + m->dev_copy.bytes;
     return TSL_OK;
 }
 

@@ -482,12 +482,15 @@ int build(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
 int build_class_grid(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
 {
     const int rc = build(m, grid_occ, init_code);
-    if (rc != TSL_ERR_OUT_OF_MEMORY) return rc;
-    // no room beside the map: it is scored without
-    (void)hipGetLastError();
-    clear_error();
-    m->grid = DevGrid{};
-    for (DevBuf* b : {&m->grid_axis, &m->grid_bits, &m->grid_cells, &m->grid_palette}) b->release();
+    if (rc == TSL_ERR_OUT_OF_MEMORY) {  // no room beside the map: it is scored without
+        (void)hipGetLastError();
+        clear_error();
+        m->grid = DevGrid{};
+    } else if (rc != TSL_OK) {
+        return rc;
+    }
+    if (!m->grid.ready)
+        for (DevBuf* b : {&m->grid_axis, &m->grid_bits, &m->grid_cells, &m->grid_palette}) b->release();
     return TSL_OK;
 }
 
