@@ -166,7 +166,9 @@ float tsl_likelihood_init(float sigma);
 /* Device bytes held by the map: voxels, lookup tables and, where the map is
  * scored through one, its class grid (the dense copy of its allocated blocks'
  * neighbourhood that the scoring kernels read; at most 4 x data_size + 32M
- * cells of 2 or 4 bytes, below 4 GB).  A server's budget starts from them. */
+ * cells of 2 or 4 bytes, below 4 GB, and no more than an eighth of the memory
+ * that is free when the map is loaded: with less free the map is scored
+ * without one, with the same weights).  A server's budget starts from them. */
 int tsl_map_device_bytes(const tsl_map* map, uint64_t* bytes);
 
 int tsl_map_destroy(tsl_map* map);

@@ -61,3 +61,19 @@ assert s.stats()["used_bytes"] == held
 s.close()
 """)
     print(out)
+
+
+def test_class_grid_leaves_the_device_room(stub):
+    """A class grid takes no more than an eighth of the free memory: with less
+    free, the map is loaded without one and filters keep the room."""
+    run(stub, """
+m = host_map()
+full = m.device_map().device_bytes()
+grid = full - 2 * m.dataSize()
+for times in (4, 12):  # what is free once the voxels are loaded, in class grids
+    m = host_map()
+    stub.stub_set_total(stub.stub_live_bytes() + 2 * m.dataSize() + times * grid)
+    d = m.device_map()
+    assert (d.device_bytes() == full) == (times == 12), (times, d.device_bytes(), full)
+    tsl.DeviceFilter(tsl.TSDFEvaluator(m), int(0.85 * times * grid) // 120)  # 116 bytes a particle
+""")

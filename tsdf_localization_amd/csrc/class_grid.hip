@@ -376,6 +376,20 @@ __global__ void k_grid_bits(const uint8_t* __restrict__ flags, uint64_t bricks, 
     bits[b] = (uint8_t)v;
 }
 
+// The dense array is a map's second copy and may be larger than the first: it
+// takes at most an eighth of the device memory that is free beside the map, so
+// that on a card that is nearly full the rest goes to filters, robots and other
+// maps as if there were no class grid.
+bool leaves_room(uint64_t bytes)
+{
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return bytes <= free_bytes / 8;
+}
+
 int build(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
 {
     const tsl_map_coef& c = m->coef;
@@ -391,6 +405,7 @@ int build(tsl_map* m, const int32_t* grid_occ, uint32_t init_code)
     const std::vector<ClassDesc>* coords = ct.coords;
     const uint32_t* pages = ct.pages;
     const uint64_t elems = ct.elems;
+    if (!leaves_room(elems * esize)) return TSL_OK;
     g.scale = ct.scale;
     for (int a = 0; a < 3; ++a) {
         g.off[a] = ct.off[a];
