@@ -25,7 +25,7 @@ std::recursive_mutex mu;
 std::map<const char*, size_t> device, pinned;
 std::vector<Copy> queue;
 size_t total = (size_t)288 << 30, live = 0;
-long launches_left = -1;  // launches until one fails (-1: none does)
+long launches_left = -1, copies_left = -1;  // launches, asynchronous copies until one fails (-1: none does)
 hipError_t last = hipSuccess;
 
 hipError_t note(hipError_t e)
@@ -56,7 +56,8 @@ extern "C" {
 
 size_t stub_live_bytes() { LOCK; return live; }
 void stub_set_total(size_t bytes) { LOCK; total = bytes; }
-void stub_fail_launch(long after) { LOCK; launches_left = after; }
+void stub_fail_launch(long after) { LOCK; launches_left = after; last = hipSuccess; }
+void stub_fail_copy(long after) { LOCK; copies_left = after; last = hipSuccess; }
 // queued copies that read or write the caller's memory
 int stub_pending()
 {
@@ -144,6 +145,11 @@ hipError_t hipGetSymbolAddress(void** p, const void*)
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t)
 {
     LOCK;
+    if (copies_left == 0) {
+        copies_left = -1;
+        return note(hipErrorUnknown);
+    }
+    if (copies_left > 0) --copies_left;
     if (kind == hipMemcpyDeviceToDevice) {
         drain();
         std::memcpy(dst, src, n);

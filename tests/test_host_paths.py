@@ -15,7 +15,7 @@ import ctypes, sys
 stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before libtsl.so
 stub.stub_live_bytes.restype = ctypes.c_size_t
 stub.stub_set_total.argtypes = [ctypes.c_size_t]
-stub.stub_fail_launch.argtypes = [ctypes.c_long]
+stub.stub_fail_launch.argtypes = stub.stub_fail_copy.argtypes = [ctypes.c_long]
 import numpy as np
 import tsdf_localization_amd as tsl
 
@@ -76,4 +76,47 @@ for times in (4, 12):  # what is free once the voxels are loaded, in class grids
     d = m.device_map()
     assert (d.device_bytes() == full) == (times == 12), (times, d.device_bytes(), full)
     tsl.DeviceFilter(tsl.TSDFEvaluator(m), int(0.85 * times * grid) // 120)  # 116 bytes a particle
+""")
+
+
+@pytest.mark.parametrize("call", ["evaluate", "evaluate_cloud", "set_scan", "set_scan_raw"])
+@pytest.mark.parametrize("step", ["launch", "copy"])
+def test_failed_call_leaves_no_copy_of_the_callers_arrays(stub, call, step):
+    """Whichever launch or copy of a call fails, when it returns no queued copy
+    reads or writes the caller's arrays (large enough not to be staged)."""
+    run(stub, f"""
+ev = tsl.TSDFEvaluator(host_map())
+f = tsl.DeviceFilter(ev, 16)
+pts = np.ones((30000, 3), np.float32)
+rings = np.zeros(30000, np.int16)
+parts = np.ones((20000, 7), np.float32)
+tf = np.eye(4, dtype=np.float32)
+calls = dict(evaluate=lambda: ev.evaluate(parts, pts, tf), evaluate_cloud=lambda: ev.evaluate_cloud(parts, pts, rings, tf),
+             set_scan=lambda: f.set_scan(pts, tf), set_scan_raw=lambda: f.set_scan_raw(pts, rings, tf, 0.064))
+fail = stub.stub_fail_{step}
+for after in range(100):
+    fail(after)
+    try:
+        calls["{call}"]()
+        fail(-1)
+        break
+    except RuntimeError:
+        assert stub.stub_pending() == 0, after
+assert 0 < after < 100
+assert stub.stub_pending() == 0
+""")
+
+
+def test_call_out_of_memory_leaves_no_copy_of_the_callers_arrays(stub):
+    """The same where the particles find no device memory after the scan has
+    been queued."""
+    run(stub, """
+ev = tsl.TSDFEvaluator(host_map())
+ev.evaluate(np.ones((16, 7), np.float32), np.ones((30000, 3), np.float32), np.eye(4, dtype=np.float32))
+stub.stub_set_total(stub.stub_live_bytes())
+try:
+    ev.evaluate(np.ones((20000, 7), np.float32), np.ones((30000, 3), np.float32), np.eye(4, dtype=np.float32))
+    raise SystemExit("did not fail")
+except RuntimeError:
+    assert stub.stub_pending() == 0
 """)

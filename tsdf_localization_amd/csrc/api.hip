@@ -111,13 +111,15 @@ static char* stage_take(tsl_filter* f, size_t n)
     return p;
 }
 
-// A call that ends early waits for the copies it has queued: they may still
-// read the caller's arrays.
-static int wait_on_error(int rc)
-{
-    if (rc != TSL_OK) (void)hipDeviceSynchronize();
-    return rc;
-}
+// A call that returns between its first copy and its wait for all of them waits
+// for the copies it has queued: they may still read the caller's arrays.
+struct QueuedCopies {
+    bool pending = true;
+    ~QueuedCopies()
+    {
+        if (pending) (void)hipDeviceSynchronize();
+    }
+};
 
 static int stage_in(tsl_filter* f, void* dst, const void* src, size_t n, hipStream_t s)
 {
@@ -946,11 +948,13 @@ int tsl_filter_set_scan(tsl_filter* f, const tsl_point* pts, size_t n, const flo
     TSL_HIP_CHECK(hipDeviceSynchronize());
     TSL_TRY(filter_reserve_points(f, n));
     stage_begin(f);
+    QueuedCopies copies;
     if (n) TSL_TRY(stage_in(f, f->points_in.ptr, pts, sizeof(tsl_point) * n, 0));
     f->num_points = n;
     std::memcpy(f->tf, tf, sizeof(float) * 16);
-    TSL_TRY(wait_on_error(launch_prep_points(f, 0)));
+    TSL_TRY(launch_prep_points(f, 0));
     TSL_HIP_CHECK(hipDeviceSynchronize());
+    copies.pending = false;
     stage_begin(f);
     return TSL_OK;
 }
@@ -1309,9 +1313,8 @@ static int evaluate_filter_scan(tsl_evaluator* ev, tsl_filter* f, tsl_particle* 
             return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
         f->weights_host_cap = P;
     }
-    // (an earlier call on this filter that failed may have left its copies)
-    if (f->stage_used) TSL_HIP_CHECK(hipStreamSynchronize(s));
     stage_begin(f);
+    QueuedCopies copies;
     if (points) {
         TSL_TRY(filter_reserve_points(f, N));
         TSL_TRY(stage_in(f, f->points_in.ptr, points, sizeof(tsl_point) * N, s));
@@ -1330,6 +1333,7 @@ static int evaluate_filter_scan(tsl_evaluator* ev, tsl_filter* f, tsl_particle* 
     TSL_HIP_CHECK(hipMemcpyAsync(hs, f->state.ptr, sizeof(FilterState), hipMemcpyDeviceToHost, s));
     TSL_HIP_CHECK(hipMemcpyAsync(f->weights_host, f->raw.ptr, sizeof(float) * P, hipMemcpyDeviceToHost, s));
     TSL_HIP_CHECK(hipStreamSynchronize(s));
+    copies.pending = false;
     stage_begin(f);
     f->count_bound = hs->count;
     pose_from_stats(hs->stats, out_pose);
@@ -1439,14 +1443,15 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     TSL_TRY(f->raw_ring.reserve(ring_room + 16));  // rings, then three aligned counters
     uint32_t* counters = reinterpret_cast<uint32_t*>(f->raw_ring.as<char>() + ring_room);
     uint32_t host[3] = {0u, 0u, 0u};
+    QueuedCopies copies;
     if (n) {
         stage_begin(f);
         char* result = stage_take(f, sizeof(host));
         if (!result) return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
         TSL_TRY(stage_in(f, f->raw_in.ptr, raw, sizeof(tsl_point) * n, 0));
-        TSL_TRY(wait_on_error(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0)));
-        TSL_TRY(wait_on_error(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
-                                                 f->points_in.as<tsl_point>(), counters, 0)));
+        TSL_TRY(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0));
+        TSL_TRY(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
+                                   f->points_in.as<tsl_point>(), counters, 0));
         TSL_HIP_CHECK(hipMemcpyAsync(result, counters, sizeof(host), hipMemcpyDeviceToHost, 0));
         TSL_HIP_CHECK(hipStreamSynchronize(0));
         std::memcpy(host, result, sizeof(host));
@@ -1457,8 +1462,9 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     if (host[1]) return set_error(TSL_ERR_INVALID_ARGUMENT, "a kept point's ring is outside [0, 64)");
     f->num_points = host[0];
     std::memcpy(f->tf, tf, sizeof(float) * 16);
-    TSL_TRY(wait_on_error(launch_prep_points(f, 0)));
+    TSL_TRY(launch_prep_points(f, 0));
     TSL_HIP_CHECK(hipDeviceSynchronize());
+    copies.pending = false;
     stage_begin(f);
     return TSL_OK;
 }
