@@ -27,6 +27,7 @@ std::vector<Copy> queue;
 size_t total = (size_t)288 << 30, live = 0;
 long launches_left = -1, copies_left = -1;  // launches, asynchronous copies until one fails (-1: none does)
 hipError_t last = hipSuccess;
+bool no_pinned = false;
 
 hipError_t note(hipError_t e)
 {
@@ -58,6 +59,7 @@ size_t stub_live_bytes() { LOCK; return live; }
 void stub_set_total(size_t bytes) { LOCK; total = bytes; }
 void stub_fail_launch(long after) { LOCK; launches_left = after; last = hipSuccess; }
 void stub_fail_copy(long after) { LOCK; copies_left = after; last = hipSuccess; }
+void stub_no_pinned(int on) { LOCK; no_pinned = on != 0; }
 // queued copies that read or write the caller's memory
 int stub_pending()
 {
@@ -121,6 +123,7 @@ hipError_t hipFree(void* p)
 hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
     LOCK;
+    if (no_pinned) return note(hipErrorOutOfMemory);
     *p = std::calloc(n ? n : 1, 1);
     pinned[static_cast<char*>(*p)] = n;
     return hipSuccess;

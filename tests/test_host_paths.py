@@ -120,3 +120,15 @@ try:
 except RuntimeError:
     assert stub.stub_pending() == 0
 """)
+
+
+def test_scan_setters_without_pinned_staging(stub):
+    """A filter whose staging finds no pinned memory copies without it."""
+    run(stub, """
+f = tsl.DeviceFilter(tsl.TSDFEvaluator(host_map()), 16)
+stub.stub_no_pinned(1)
+tf = np.eye(4, dtype=np.float32)
+f.set_scan(np.ones((100, 3), np.float32), tf)
+f.set_scan_raw(np.ones((100, 3), np.float32), np.zeros(100, np.int16), tf, 0.064)
+f.get_particles()
+""")

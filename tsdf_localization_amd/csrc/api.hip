@@ -1447,14 +1447,14 @@ static int set_scan_reduced(tsl_filter* f, int mode, const tsl_point* raw, const
     if (n) {
         stage_begin(f);
         char* result = stage_take(f, sizeof(host));
-        if (!result) return set_error(TSL_ERR_OUT_OF_MEMORY, "hipHostMalloc failed");
         TSL_TRY(stage_in(f, f->raw_in.ptr, raw, sizeof(tsl_point) * n, 0));
         TSL_TRY(stage_in(f, f->raw_ring.ptr, ring, ring_bytes * n, 0));
         TSL_TRY(launch_reduce_scan(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
                                    f->points_in.as<tsl_point>(), counters, 0));
-        TSL_HIP_CHECK(hipMemcpyAsync(result, counters, sizeof(host), hipMemcpyDeviceToHost, 0));
+        TSL_HIP_CHECK(hipMemcpyAsync(result ? static_cast<void*>(result) : host, counters, sizeof(host),
+                                     hipMemcpyDeviceToHost, 0));
         TSL_HIP_CHECK(hipStreamSynchronize(0));
-        std::memcpy(host, result, sizeof(host));
+        if (result) std::memcpy(host, result, sizeof(host));
         if (host[2])
             TSL_TRY(launch_reduce_order(f, mode, f->raw_in.as<tsl_point>(), f->raw_ring.ptr, (uint32_t)n, cell,
                                         f->points_in.as<tsl_point>(), counters, 0));
