@@ -292,8 +292,8 @@ int tsl_check_magic_divisor(uint32_t divisor, uint32_t stride, uint64_t* mismatc
 
 /* Self-check of the class grid the scoring kernels read a map through, host
  * only: the voxel index its tables give for n transformed points t (x, y, z in
- * map coordinates, |t| < 2^22) -- coef->data_size where init_value is read,
- * UINT64_MAX where the lookup is left to the exact tiers.  *has_grid = 0 (and
+ * map coordinates) -- coef->data_size where init_value is read, UINT64_MAX
+ * where the lookup is left to the exact tiers (all |t| >= 2^22 among them).  *has_grid = 0 (and
  * nothing written) if the map has none.  No counterpart in the reference. */
 int tsl_check_class_grid(const tsl_map_coef* coef, const int32_t* grid_occ, const float* t, size_t n,
                          uint64_t* index, int* has_grid);

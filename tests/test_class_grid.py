@@ -4,6 +4,9 @@ points inside, on and next to every class boundary, below and above the map,
 for maps of even and odd sub_dim, offsets that reach into other blocks, and
 extents that end inside a block; and the maps that have no class grid."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -95,3 +98,35 @@ def test_class_grid_index_is_the_references(name):
     inside = ((t - lo) > -1.0).all(1)
     assert not left[inside].any()
     assert np.count_nonzero(ref[inside] < c.data_size) > 1000
+
+
+@pytest.mark.parametrize("field,value", [("up_dim_2", 0), ("resolution", -1.0), ("sub_dim_2", 7), ("grid_occ_size", 0)])
+def test_inconsistent_coefficients_are_refused(field, value):
+    """As tsl_map_create refuses them, in a process of its own: a zero
+    up_dim_2 was a division by zero."""
+    code = f"""
+import ctypes
+import numpy as np
+import tsdf_localization_amd as tsl
+from tsdf_localization_amd import _lib
+c = tsl.coef_init((0, 0, 0), (3, 3, 3), 0.05)
+grid = np.zeros(int(c.grid_occ_size), np.int32)
+c.data_size = int(c.sub_dim) ** 3
+c.{field} = {value}
+has = ctypes.c_int()
+rc = _lib.lib.tsl_check_class_grid(ctypes.byref(c), _lib.ptr(grid), None, 0, None, ctypes.byref(has))
+assert rc == _lib.TSL_ERR_INVALID_ARGUMENT, rc
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stderr)
+
+
+def test_coordinates_out_of_range_are_left_to_the_exact_tiers():
+    c, grid, _ = _case("even")
+    t = np.array([[np.nan, 1, 1], [1, np.inf, 1], [1, 1, -np.inf], [4194304.0, 1, 1]], np.float32)
+    got = np.zeros(4, np.uint64)
+    has = ctypes.c_int()
+    _lib.check(_lib.lib.tsl_check_class_grid(ctypes.byref(c), _lib.ptr(grid), _lib.ptr(t), 4, _lib.ptr(got),
+                                             ctypes.byref(has)))
+    assert has.value == 1 and np.all(got == EXACT)

@@ -208,6 +208,20 @@ void pose_from_stats(const double* st, tsl_pose* pose)
     pose->orientation[3] = cr * cp * cy + sr * sp * sy;
 }
 
+int validate_coef(const tsl_map_coef* c)
+{
+    if (!(c->resolution > 0.0f) || !std::isfinite(c->resolution))
+        return set_error(TSL_ERR_INVALID_ARGUMENT, "resolution must be positive and finite");
+    if (c->grid_occ_size != c->up_dim_x * c->up_dim_y * c->up_dim_z || c->grid_occ_size == 0)
+        return set_error(TSL_ERR_INVALID_ARGUMENT, "grid_occ_size does not match the block dims");
+    if (c->up_dim_2 != c->up_dim_x * c->up_dim_y || c->sub_dim_2 != c->sub_dim * c->sub_dim)
+        return set_error(TSL_ERR_INVALID_ARGUMENT, "inconsistent derived dims");
+    if (c->data_size > 0x7fffffffull || c->grid_occ_size > 0x7fffffffull || c->sub_dim > 1024)
+        return set_error(TSL_ERR_UNSUPPORTED, "map exceeds the int32 block table of the reference (%llu voxels)",
+                         (unsigned long long)c->data_size);
+    return TSL_OK;
+}
+
 }  // namespace tsl
 
 using namespace tsl;
@@ -255,20 +269,6 @@ int tsl_map_coef_init(float min_x, float min_y, float min_z, float max_x, float 
     c->sub_dim_2 = c->sub_dim * c->sub_dim;
     c->grid_occ_size = c->up_dim_x * c->up_dim_y * c->up_dim_z;
     c->data_size = 0;
-    return TSL_OK;
-}
-
-static int validate_coef(const tsl_map_coef* c)
-{
-    if (!(c->resolution > 0.0f) || !std::isfinite(c->resolution))
-        return set_error(TSL_ERR_INVALID_ARGUMENT, "resolution must be positive and finite");
-    if (c->grid_occ_size != c->up_dim_x * c->up_dim_y * c->up_dim_z || c->grid_occ_size == 0)
-        return set_error(TSL_ERR_INVALID_ARGUMENT, "grid_occ_size does not match the block dims");
-    if (c->up_dim_2 != c->up_dim_x * c->up_dim_y || c->sub_dim_2 != c->sub_dim * c->sub_dim)
-        return set_error(TSL_ERR_INVALID_ARGUMENT, "inconsistent derived dims");
-    if (c->data_size > 0x7fffffffull || c->grid_occ_size > 0x7fffffffull || c->sub_dim > 1024)
-        return set_error(TSL_ERR_UNSUPPORTED, "map exceeds the int32 block table of the reference (%llu voxels)",
-                         (unsigned long long)c->data_size);
     return TSL_OK;
 }
 

@@ -517,6 +517,7 @@ extern "C" int tsl_check_class_grid(const tsl_map_coef* coef, const int32_t* gri
     using namespace tsl;
     if (!coef || !grid_occ || !has_grid || (n && (!t || !index)))
         return set_error(TSL_ERR_INVALID_ARGUMENT, "NULL argument");
+    TSL_TRY(validate_coef(coef));
     const tsl_map_coef& c = *coef;
     const uint32_t gthr[3] = {grid_threshold(c.dim_x, c.resolution), grid_threshold(c.dim_y, c.resolution),
                               grid_threshold(c.dim_z, c.resolution)};
@@ -527,13 +528,18 @@ extern "C" int tsl_check_class_grid(const tsl_map_coef* coef, const int32_t* gri
     negative_band_constants(c, fm);
     const uint64_t neg[3] = {fm.neg_x, fm.neg_y, fm.neg_z};
     for (size_t i = 0; i < n; ++i) {
+        const float* p = t + 3 * i;
+        if (!(std::fabs(p[0]) < 4194304.0f && std::fabs(p[1]) < 4194304.0f && std::fabs(p[2]) < 4194304.0f)) {
+            index[i] = ~0ull;
+            continue;
+        }
         uint32_t addr = 0;
         for (int a = 0; a < 3; ++a) {
-            const float v = std::min(std::max(std::fmaf(t[3 * i + a], ct.scale, ct.off[a]), kGridMagic), ct.top[a]);
+            const float v = std::min(std::max(std::fmaf(p[a], ct.scale, ct.off[a]), kGridMagic), ct.top[a]);
             const AxisEntry& e = ct.table[ct.first[a] + (uint32_t)(v - kGridMagic)];
             float edge;
             std::memcpy(&edge, &e.thr, 4);
-            addr += t[3 * i + a] >= edge ? e.c_hi : e.c_lo;
+            addr += p[a] >= edge ? e.c_hi : e.c_lo;
         }
         uint32_t x, y, z;
         grid_coord(addr / 2, ct.pages[0], ct.pages[1], x, y, z);

@@ -243,6 +243,8 @@ constexpr size_t kGridLdsBudget = 80 << 10;  // two workgroups of 16 wavefronts 
 
 // Smallest u in [0, 2^23] with trunc(fl(fl(u)/res)) >= dim; host IEEE division.
 uint32_t grid_threshold(uint64_t dim, float res);
+// An error where a map's coefficients contradict each other or exceed the int32 form.
+int validate_coef(const tsl_map_coef* c);
 // Bound R of |offset| that keeps every block index of the 32-bit tiers in int32.
 float lookup_range(const tsl_map_coef& c);
 
