@@ -132,3 +132,22 @@ f.set_scan(np.ones((100, 3), np.float32), tf)
 f.set_scan_raw(np.ones((100, 3), np.float32), np.zeros(100, np.int16), tf, 0.064)
 f.get_particles()
 """)
+
+
+def test_wide_map_evaluates_as_many_items_as_with_two_particles(stub):
+    """The 64-bit form's automatic tile (one particle per wavefront) refuses no
+    particles x chunks that two per wavefront can launch."""
+    run(stub, """
+c = tsl.coef_init((0, 0, 0), (3.0, 3.0, 2.0), 0.05, 0.25)
+n, sd3 = int(c.grid_occ_size), int(c.sub_dim) ** 3
+c.data_size = n * sd3
+m = tsl.CudaSubVoxelMap(c, np.arange(n, dtype=np.int64) * sd3, tsdf_mm=np.zeros(n * sd3, np.int16), truncation_mm=300,
+                        sigma=0.1)
+P, N = 230_000, 64 * 40_000
+f = tsl.DeviceFilter(tsl.TSDFEvaluator(m), P)
+f.set_particles(np.ones((P, 7), np.float32))
+f.set_scan(np.ones((N, 3), np.float32), np.eye(4, dtype=np.float32))
+assert 2 ** 31 < (P + 3) // 4 * (N // 64) < 2 ** 32
+f.set_tile(0, 64, 0)
+f.update_async()
+""")

@@ -427,6 +427,13 @@ __global__ void k_restore(const tsl_particle* __restrict__ src, tsl_particle* __
 // point chunks to give the 256 CUs at least four full rounds of wavefronts.
 }  // namespace
 
+// Workgroups of an evaluation launch, and the most a launch may have.
+static size_t eval_items(const Tile& t, size_t P)
+{
+    return ((P + t.K - 1) / t.K + kWaves - 1) / kWaves * t.chunks;
+}
+constexpr size_t kMaxEvalItems = 0x7fffffffull;
+
 Tile choose_tile(const tsl_filter* f, size_t P, size_t N)
 {
     Tile t;
@@ -458,6 +465,8 @@ Tile choose_tile(const tsl_filter* f, size_t P, size_t N)
     t.chunk_len = (uint32_t)len;
     t.chunks = (uint32_t)((N + len - 1) / len);
     if (t.chunks == 0) t.chunks = 1;
+    // (twice the particles a workgroup where the launch would hold too many)
+    if (!f->tile_k && t.K == 1 && eval_items(t, P) > kMaxEvalItems) t.K = 2;
     return t;
 }
 
@@ -480,9 +489,8 @@ int launch_eval_kernel(const Tile& tile, const tsl_filter* f, size_t P, size_t N
                        float* partial, void* trace_out)
 {
     const tsl_map* map = f->ev->map;
-    const size_t groups = (P + tile.K - 1) / tile.K;
-    const size_t items = (groups + kWaves - 1) / kWaves * tile.chunks;
-    if (items > 0x7fffffffull) return set_error(TSL_ERR_UNSUPPORTED, "evaluation grid too large");
+    const size_t items = eval_items(tile, P);
+    if (items > kMaxEvalItems) return set_error(TSL_ERR_UNSUPPORTED, "evaluation grid too large");
     // (the class grid holds values, not the reference's indices)
     if (kMode != 1 && tile.grid) return launch_grid(kMode, f, tile, P, N, stream, partial, trace_out);
     const dim3 grid((unsigned)items);
