@@ -413,8 +413,9 @@ int tsl_filter_set_block_lookup(tsl_filter* f, int mode);
  * tile) on the filter's current particles and scan (reps launches each, on
  * `stream`, synchronously) and keep the fastest; reports it through the
  * non-NULL out arguments (best_ms: evaluation kernel plus the per-update
- * cost of the particle order).  No counterpart in the reference (its launch
- * shape is fixed, src/cuda/cuda_evaluator.cu:301). */
+ * cost of the particle order).  On a class grid the candidates are particle
+ * order x chunks.  No counterpart in the reference (its launch shape is
+ * fixed, src/cuda/cuda_evaluator.cu:301). */
 int tsl_filter_autotune(tsl_filter* f, void* stream, int reps, int* best_order, int* best_k,
                         int* best_points_per_lane, uint32_t* best_chunk, float* best_ms);
 
@@ -480,7 +481,8 @@ int tsl_batch_set_tile(tsl_batch* b, int k, int points_per_lane, uint32_t chunk_
 /* Time the batched update (every member, reps launches per candidate on
  * `stream`, synchronously) for every tile k in {1, 2} x points per lane in
  * {1, 2, 4} x chunk_len in {automatic, 1024, 4096, 8192} and keep the
- * fastest (tsl_batch_set_tile); reports it through the non-NULL out
+ * fastest (tsl_batch_set_tile; on a class grid only chunk_len is timed, k and
+ * points per lane stay as they are); reports it through the non-NULL out
  * arguments.  Leaves every member as one update would (weights
  * normalised, particles and counts unchanged).  No counterpart in the
  * reference (one filter per process, fixed launch shape,

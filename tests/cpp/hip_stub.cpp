@@ -28,6 +28,7 @@ size_t total = (size_t)288 << 30, live = 0;
 long launches_left = -1, copies_left = -1;  // launches, asynchronous copies until one fails (-1: none does)
 hipError_t last = hipSuccess;
 bool no_pinned = false;
+int timings = 0;
 
 hipError_t note(hipError_t e)
 {
@@ -60,6 +61,8 @@ void stub_set_total(size_t bytes) { LOCK; total = bytes; }
 void stub_fail_launch(long after) { LOCK; launches_left = after; last = hipSuccess; }
 void stub_fail_copy(long after) { LOCK; copies_left = after; last = hipSuccess; }
 void stub_no_pinned(int on) { LOCK; no_pinned = on != 0; }
+// event pairs measured since the last call
+int stub_timings() { LOCK; const int n = timings; timings = 0; return n; }
 // queued copies that read or write the caller's memory
 int stub_pending()
 {
@@ -188,7 +191,7 @@ hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { LOCK; drain(); return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { LOCK; drain(); return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { LOCK; ++timings; *ms = 1.0f; return hipSuccess; }
 
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*) { std::memset(a, 0, sizeof(*a)); return hipSuccess; }

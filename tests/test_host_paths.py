@@ -151,3 +151,25 @@ assert 2 ** 31 < (P + 3) // 4 * (N // 64) < 2 ** 32
 f.set_tile(0, 64, 0)
 f.update_async()
 """)
+
+
+@pytest.mark.parametrize("res,filter_shapes,batch_shapes", [(0.05, 6, 4), (0.04, 60, 24)])
+def test_autotuners_time_each_distinct_shape_once(stub, res, filter_shapes, batch_shapes):
+    """On a class grid (0.05 m) neither K nor points per lane shapes the kernel:
+    what differs are the chunks (five lengths, the automatic one by K; a
+    batch's four).  Without one (0.04 m): two lookups x six shapes x five
+    lengths, a batch's six shapes x four.  Each in both particle orders, whose
+    own time is measured too."""
+    run(stub, f"""
+ev = tsl.TSDFEvaluator(host_map(res={res}))
+f = tsl.DeviceFilter(ev, 64)
+f.set_particles(np.ones((64, 7), np.float32))
+f.set_scan(np.ones((5000, 3), np.float32), np.eye(4, dtype=np.float32))
+stub.stub_timings()
+f.autotune(reps=1)
+assert stub.stub_timings() == 2 * (1 + {filter_shapes})
+b = tsl.Batch(ev, [f])
+b.set_tile(1, 0, 4)
+k, pp, chunk, ms = b.autotune(tsl.Stream(), reps=1)
+assert stub.stub_timings() == {batch_shapes}
+""")

@@ -259,11 +259,13 @@ int tsl_batch_autotune(tsl_batch* b, void* stream, int reps, int* best_k, int* b
     int bk = saved_k, bp = saved_p;
     uint32_t bc = saved_chunk;
     int rc = TSL_OK;
-    for (int ki = 0; ki < 2 && rc == TSL_OK; ++ki)
-        for (int pi = 0; pi < 3 && rc == TSL_OK; ++pi)
+    // (a class grid's kernel has one shape: the chunks are what differs)
+    const bool grid = b->ev->map->grid.ready != 0;
+    for (int ki = 0; ki < (grid ? 1 : 2) && rc == TSL_OK; ++ki)
+        for (int pi = 0; pi < (grid ? 1 : 3) && rc == TSL_OK; ++pi)
             for (int ci = 0; ci < 4 && rc == TSL_OK; ++ci) {
-                b->K = ks[ki];
-                b->P = ps[pi];
+                b->K = grid ? saved_k : ks[ki];
+                b->P = grid ? saved_p : ps[pi];
                 b->chunk_len = chunks[ci];
                 rc = prepare(b);
                 if (rc == TSL_OK) rc = enqueue_step(b, false, false, s);  // warm-up

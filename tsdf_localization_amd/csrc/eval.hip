@@ -618,7 +618,8 @@ static int launch_eval_core(tsl_filter* f, hipStream_t stream, Tile& tile)
 // Time every candidate tile shape on the current particles and scan; keep
 // the fastest.  Candidates: particle order {caller, spatial} x block lookup
 // x K in {1, 2} x points per lane in {1, 2, 4} x {automatic chunks, 1/2/4/8
-// chunks of the scan}.  A candidate's time is its evaluation kernel plus the
+// chunks of the scan}; on a class grid, whose kernel has one shape, particle
+// order x chunks (the automatic ones for both K).  A candidate's time is its evaluation kernel plus the
 // per-update cost of its particle order (pose matrices, and for the spatial
 // order the key computation and sort).
 int autotune_tile(tsl_filter* f, hipStream_t stream, int reps, int* best_order, int* best_k, int* best_p,
@@ -640,7 +641,9 @@ int autotune_tile(tsl_filter* f, hipStream_t stream, int reps, int* best_order, 
     const uint32_t div[5] = {0, 1, 2, 4, 8};
     int rc = TSL_OK;
     // a class grid has neither a block table nor a rank table to choose
-    const int ranks = !f->ev->map->grid.ready && f->ev->map->dev.occ_nwords ? 2 : 1;
+    const bool grid = f->ev->map->grid.ready != 0;
+    const int ranks = !grid && f->ev->map->dev.occ_nwords ? 2 : 1;
+    const int npp = grid ? 1 : 3;
     for (int order = 0; order < 2 && rc == TSL_OK; ++order) {
         f->order_mode = order;
         Tile pt = choose_tile(f, P, N);
@@ -657,8 +660,9 @@ int autotune_tile(tsl_filter* f, hipStream_t stream, int reps, int* best_order, 
         for (int rk = 0; rk < ranks && rc == TSL_OK; ++rk) {
         f->rank_mode = rk;
         for (int ki = 0; ki < 2 && rc == TSL_OK; ++ki) {
-            for (int pi = 0; pi < 3 && rc == TSL_OK; ++pi) {
+            for (int pi = 0; pi < npp && rc == TSL_OK; ++pi) {
                 for (int ci = 0; ci < 5 && rc == TSL_OK; ++ci) {
+                    if (grid && div[ci] && ki == 0) continue;
                     f->tile_k = ks[ki];
                     f->tile_p = ps[pi];
                     f->tile_chunk = div[ci] ? (uint32_t)((N + div[ci] - 1) / div[ci]) : 0u;
