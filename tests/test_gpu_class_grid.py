@@ -4,6 +4,8 @@ additions of non-negative terms, 2^-24 each), for palette and float forms, at
 the remainders of particles and points, with lanes in the thin classes below
 the map, lanes and points left to the exact tiers, and matrices out of their
 range."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -71,3 +73,40 @@ def test_scan_ending_on_an_allocation_boundary(N):
     tf = np.ascontiguousarray(np.eye(4, dtype=np.float32).reshape(-1))
     _, w64 = ob.OracleMap(c, grid, data).evaluate(parts, pts, tf)
     assert np.max(rel_err(ev.evaluate_raw(parts, pts, tf), w64)) <= 524 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("form", ["palette", "float"])
+def test_coarse_granules(form):
+    """A map whose bitmap fits the LDS only with granules of several bricks (67
+    million class triples: 512 B for 16-bit cells, 1 KB for floats), one voxel in
+    300 holding a value, so that most granules that are read hold few."""
+    import tsdf_localization_amd as tsl
+    from tsdf_localization_amd import _lib
+    c = tsl.coef_init((0.0, 0.0, 0.0), (30.0, 30.0, 8.0), 0.05)
+    c.init_value = 0.0126
+    rng = np.random.default_rng(3)
+    n, sd3 = int(c.grid_occ_size), int(c.sub_dim) ** 3
+    alloc = rng.uniform(size=n) < 0.3
+    alloc[n - 1] = True
+    grid = np.where(alloc, (np.cumsum(alloc) - 1) * sd3, -1).astype(np.int32)
+    size = c.data_size = int(alloc.sum()) * sd3
+    data = np.full(size, np.float32(c.init_value))
+    at = rng.integers(0, size, size // 300)
+    data[at] = np.resize(rng.uniform(0.01, 1.0, 300 if form == "palette" else at.size).astype(np.float32), at.size)
+    has = ctypes.c_int()
+    _lib.check(_lib.lib.tsl_check_class_grid(ctypes.byref(c), _lib.ptr(grid), None, 0, None, ctypes.byref(has)))
+    assert has.value == 1
+    ev = tsl.TSDFEvaluator(tsl.CudaSubVoxelMap(c, grid, data=data))
+    om = ob.OracleMap(c, grid, data)
+    parts = np.zeros((300, 7), np.float32)
+    parts[:, :3] = rng.uniform(0.0, 1.0, (300, 3)) * (30, 30, 8)
+    parts[:, 3:6] = rng.uniform(-3.1, 3.1, (300, 3))
+    parts[:, 6] = 1.0 / 300
+    pts = rng.uniform(-6.0, 6.0, (1500, 3)).astype(np.float32)
+    tf = np.ascontiguousarray(np.eye(4, dtype=np.float32).reshape(-1))
+    ref = oracle_values(om, om.trace(parts, pts, tf))
+    assert np.count_nonzero(ref != np.float32(c.init_value)) > 100
+    got = ev.trace_values(parts, pts, tf)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    _, w64 = om.evaluate(parts, pts, tf)
+    assert np.max(rel_err(ev.evaluate_raw(parts, pts, tf), w64)) <= WEIGHT_RTOL

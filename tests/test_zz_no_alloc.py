@@ -137,3 +137,19 @@ def test_noalloc_other_map_forms(tsl, room):
             assert rc == 0, tsl._lib.lib.tsl_last_error()
             want = ev.evaluate_raw(parts, pts, room.tf)
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), name
+
+
+@pytest.mark.parametrize("P", [8191, 8192, 1_000_000, 1_060_000])
+def test_noalloc_at_the_edges_of_the_spatial_order(tsl, room, P):
+    """Particles in the caller's order (8191), spatial order (8192, 1,000,000)
+    and, where the scratch holds no order any more, the caller's again
+    (1,060,000): the bits of tsl_evaluate_raw each time."""
+    rng = np.random.default_rng(P)
+    parts = np.resize(room.particles, (P, 7)).copy()
+    parts[:, :3] += rng.normal(0, 0.3, (P, 3)).astype(np.float32)
+    ev = tsl.TSDFEvaluator(room.map)
+    pts = room.points[:130]
+    rc, got = _noalloc(ev, parts, pts, room.tf)
+    assert rc == 0, tsl._lib.lib.tsl_last_error()
+    want = ev.evaluate_raw(parts, pts, room.tf)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
