@@ -258,8 +258,9 @@ int tsl_evaluate_raw(tsl_evaluator* ev, const tsl_particle* particles, size_t nu
  * Every intermediate lives in a fixed 64 MiB device array per GPU, which
  * the library holds until the process ends; TSL_ERR_CAPACITY if the call
  * needs more (about 52 B per particle, 60 B per point, plus 4 B per particle
- * per scan chunk; from 8192 particles, where 12 B per particle and 1 MB more
- * fit, the particles are evaluated in spatial order, with the same weights).  Enqueued on `stream` with no allocation, no host copy
+ * per scan chunk; from 8192 particles, 256 points and 2^25 pairs, where 12 B
+ * per particle and 1 MB more fit, the particles are evaluated in spatial order,
+ * with the same weights).  Enqueued on `stream` with no allocation, no host copy
  * and no synchronisation.  Calls that overlap on one GPU share the array
  * and race: serialise them (one stream, or events). */
 int tsl_evaluate_raw_noalloc(tsl_evaluator* ev, const tsl_particle* particles, size_t num_particles,

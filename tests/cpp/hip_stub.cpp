@@ -28,7 +28,7 @@ size_t total = (size_t)288 << 30, live = 0;
 long launches_left = -1, copies_left = -1;  // launches, asynchronous copies until one fails (-1: none does)
 hipError_t last = hipSuccess;
 bool no_pinned = false;
-int timings = 0;
+int timings = 0, launches = 0;
 
 hipError_t note(hipError_t e)
 {
@@ -63,6 +63,8 @@ void stub_fail_copy(long after) { LOCK; copies_left = after; last = hipSuccess; 
 void stub_no_pinned(int on) { LOCK; no_pinned = on != 0; }
 // event pairs measured since the last call
 int stub_timings() { LOCK; const int n = timings; timings = 0; return n; }
+// kernels launched since the last call
+int stub_launches() { LOCK; const int n = launches; launches = 0; return n; }
 // queued copies that read or write the caller's memory
 int stub_pending()
 {
@@ -214,6 +216,7 @@ hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t)
         return note(hipErrorLaunchFailure);
     }
     if (launches_left > 0) --launches_left;
+    ++launches;
     return hipSuccess;
 }
 

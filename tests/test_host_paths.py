@@ -173,3 +173,24 @@ b.set_tile(1, 0, 4)
 k, pp, chunk, ms = b.autotune(tsl.Stream(), reps=1)
 assert stub.stub_timings() == {batch_shapes}
 """)
+
+
+def test_spatial_order_of_the_allocation_free_entry(stub):
+    """The order's launches come only where there are pairs enough to pay for
+    them: not for short scans, nor for few pairs."""
+    run(stub, """
+ev = tsl.TSDFEvaluator(host_map())
+tf = np.eye(4, dtype=np.float32)
+tf_p = ctypes.c_void_p(tf.ctypes.data)
+def launches(P, N):
+    p, q, w = np.ones((P, 7), np.float32), np.ones((N, 3), np.float32), np.empty(P, np.float32)
+    stub.stub_launches()
+    rc = tsl._lib.lib.tsl_evaluate_raw_noalloc(ev.handle, tsl._lib.ptr(p), P, tsl._lib.ptr(q), N, tf_p,
+                                               tsl._lib.ptr(w), None)
+    assert rc == 0
+    return stub.stub_launches()
+plain = launches(1000, 300)
+for P, N, ordered in [(8191, 5000, False), (8192, 4095, False), (8192, 4096, True), (20000, 64, False),
+                      (200000, 255, False), (200000, 256, True), (100000, 335, False), (100000, 336, True)]:
+    assert (launches(P, N) > plain) == ordered, (P, N)
+""")

@@ -139,16 +139,18 @@ def test_noalloc_other_map_forms(tsl, room):
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), name
 
 
-@pytest.mark.parametrize("P", [8191, 8192, 1_000_000, 1_060_000])
-def test_noalloc_at_the_edges_of_the_spatial_order(tsl, room, P):
-    """Particles in the caller's order (8191), spatial order (8192, 1,000,000)
-    and, where the scratch holds no order any more, the caller's again
-    (1,060,000): the bits of tsl_evaluate_raw each time."""
+@pytest.mark.parametrize("P,N", [(8191, 130), (8192, 130), (8192, 4095), (8192, 4096), (200_000, 255), (200_000, 256),
+                                 (1_000_000, 130), (1_000_000, 256), (1_060_000, 256)])
+def test_noalloc_at_the_edges_of_the_spatial_order(tsl, room, P, N):
+    """Particles in the caller's order where they are fewer than 8192, the
+    points fewer than 256 or the pairs fewer than 2^25, in spatial order past
+    that and, where the scratch holds no order any more (1,060,000), in the
+    caller's again: the bits of tsl_evaluate_raw each time."""
     rng = np.random.default_rng(P)
     parts = np.resize(room.particles, (P, 7)).copy()
     parts[:, :3] += rng.normal(0, 0.3, (P, 3)).astype(np.float32)
     ev = tsl.TSDFEvaluator(room.map)
-    pts = room.points[:130]
+    pts = np.resize(room.points, (N, 3))
     rc, got = _noalloc(ev, parts, pts, room.tf)
     assert rc == 0, tsl._lib.lib.tsl_last_error()
     want = ev.evaluate_raw(parts, pts, room.tf)

@@ -26,6 +26,8 @@ namespace {
 
 constexpr size_t kScratchBytes = 64ull << 20;  // 64 MiB per device
 constexpr int kMaxDevices = 64;
+// Fewest points, and particles x points, that are evaluated in spatial order.
+constexpr size_t kOrderPoints = 256, kOrderPairs = 1ull << 25;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -114,13 +116,17 @@ extern "C" int tsl_evaluate_raw_noalloc(tsl_evaluator* ev, const tsl_particle* p
     constexpr size_t parts = sizeof(sizes) / sizeof(sizes[0]);
     size_t need = 0, order_need = 0;
     for (size_t k = 0; k < parts; ++k) (k < parts - kOrder ? need : order_need) += round256(sizes[k]);
-    // The spatial order (choose_tile's rule) where the scratch holds its 12 B
-    // per particle as well, up to about 1,030,000 particles; the caller's
-    // order beyond, with the same weights.  1,000,000 particles drawn over a
-    // building x 3989 points: 15.2 ms in spatial order against 20.1 in the
-    // caller's, whose particles share no cache lines (9.1 since the evaluation's
-    // wavefronts walk the scan in step).
-    tile.order = tile.order && need + order_need <= kScratchBytes;
+    // The spatial order (from 8192 particles, choose_tile's rule) where it pays
+    // for itself and the scratch holds its 12 B per particle as well, up to
+    // about 1,030,000 particles; the caller's order elsewhere, with the same
+    // weights.  Its launches cost 20 us and a share that grows with the
+    // particles, what it saves grows with the pairs, and with how far the
+    // particles are spread.  Caller's against spatial order, spread over a
+    // building: 8192 x 4000 224 and 223 us, 20,000 x 1500 241 and 223, 50,000
+    // x 300 149 and 150, 600,000 x 700 3159 and 2245; around one pose: 20,000 x
+    // 1500 159 and 170, 50,000 x 4000 672 and 647, 600,000 x 64 233 and 457,
+    // 600,000 x 700 1708 and 1781.
+    tile.order = tile.order && N >= kOrderPoints && P * N >= kOrderPairs && need + order_need <= kScratchBytes;
     f.order_mode = tile.order;
     if (need > kScratchBytes)
         return set_error(TSL_ERR_CAPACITY,
