@@ -194,3 +194,17 @@ for P, N, ordered in [(8191, 5000, False), (8192, 4095, False), (8192, 4096, Tru
                       (200000, 255, False), (200000, 256, True), (100000, 335, False), (100000, 336, True)]:
     assert (launches(P, N) > plain) == ordered, (P, N)
 """)
+
+
+def test_lone_filters_resample_in_one_launch_up_to_6144_candidates(stub):
+    run(stub, """
+ev = tsl.TSDFEvaluator(host_map())
+for n, one in [(2000, True), (2100, True), (6100, True), (6200, False), (8100, False)]:
+    f = tsl.DeviceFilter(ev, n)
+    f.set_particles(np.ones((n, 7), np.float32))
+    stub.stub_launches()
+    f.resample_async(np.float32(0.3 / n))
+    first = stub.stub_launches()
+    f.resample_async(np.float32(0.3 / n))
+    assert (stub.stub_launches() == 1) == one, (n, first)
+""")

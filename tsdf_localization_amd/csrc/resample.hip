@@ -35,10 +35,14 @@ namespace {
 
 constexpr int kRsThreads = 1024;
 // A lone filter with at most this many candidates resamples in one launch (its
-// running sum, U and weights in 128 KB of LDS).  5,000 particles: 32 us against
-// 43 in seven launches and the gaps between them.  A third of it is thread 0
-// walking the runs of U; past 8192 the LDS is too small.
-constexpr uint32_t kRsSmall = 8192;
+// running sum, U and weights in 96 KB of LDS).  A restore and a resampling, back
+// to back: 2,100 particles 23 us against 32 in seven launches, 5,000 34 against
+// 40, 6,000 36.5 against 38.5; with eight candidates a thread 7,000 42 against
+// 39 and 8,100 45 against 40 (the one workgroup then takes longer over them than
+// the launches cost).  A third of it is thread 0 walking the runs of U.
+constexpr uint32_t kRsSmall = 6144;
+constexpr int kRsSmallPer = (int)(kRsSmall / kRsThreads);
+static_assert(kRsSmall % kRsThreads == 0, "");
 
 __host__ __device__ __forceinline__ float rec_step(float u, double inv_m) { return (float)((double)u + inv_m); }
 
@@ -604,9 +608,11 @@ int launch_resample_members(Member* d_members, uint32_t n, uint32_t grid_cap, fl
         } else {
             // (more LDS than the runtime grants unasked; a host call, cheap and
             // allowed during a capture)
-            TSL_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rs_small<8>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsSmallLds<8>));
-            hipLaunchKernelGGL(k_rs_small<8>, dim3(1, 1), dim3(kRsThreads), kRsSmallLds<8>, stream, d_members, u0_arg,
+            constexpr auto kernel = &k_rs_small<kRsSmallPer>;
+            constexpr size_t lds = kRsSmallLds<kRsSmallPer>;
+            TSL_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(kernel, dim3(1, 1), dim3(kRsThreads), lds, stream, d_members, u0_arg,
                                copy_back ? 1 : 0);
         }
         TSL_HIP_CHECK(hipGetLastError());
