@@ -591,9 +591,10 @@ int tsl_server_stats(tsl_server* s, uint64_t* used_bytes, uint64_t* ticks, uint6
 /* Robots of 65,536 particle slots and more (global localisation) are served
  * on a stream of their own, apart from the others (every server of a device
  * shares the two streams), and their evaluation is cut into launches of
- * about `pairs` particle-point pairs on a grid that leaves reserved_per_cu
- * workgroup slots per compute unit free, so other requests' kernels start
- * within about one launch (default 2^27 pairs, 2 slots; pairs = 0: one
+ * about `pairs` particle-point pairs on a grid that leaves the room of
+ * reserved_per_cu four-wavefront workgroups per compute unit free (at most all
+ * but one workgroup of each), so other requests' kernels start within about one
+ * launch (default 2^27 pairs, 2 slots; pairs = 0: one
  * launch per tick on the whole grid).  Results are the same bits either way.
  * Takes effect for ticks started afterwards. */
 int tsl_server_set_slice(tsl_server* s, uint64_t pairs, uint32_t reserved_per_cu);

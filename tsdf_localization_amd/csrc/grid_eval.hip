@@ -14,8 +14,8 @@
 //
 // 100,000 particles x 20,000 points of the benchmark's building:
 // 2.57 ms against 3.84 (7.8e11 pairs/s against 5.2e11); VALU instructions issue
-// on 95 % of the cycles (2.2 ms with the gathers taken out).  Where two thirds
-// of the pairs read a cell (tracking filters) the texture-data path is full
+// on 96 % of the cycles (2.2 ms with the gathers taken out).  Where 85 to 90 % of
+// the pairs read a cell (tracking filters) the texture-data path is full
 // instead, and a million sparse particles wait for lines beyond the L2.  Two
 // particles are in flight per wavefront because more of them
 // (4, 8) put more distinct cells in flight than the L2 holds.

@@ -15,9 +15,9 @@
 // ("tracking").  Each class has its own stream and its own ticks, so a
 // tracking request never queues behind a bulk one; a bulk tick's evaluation
 // is cut into slices of a bounded number of particle-point pairs, launched
-// one after the other on a grid that leaves two workgroup slots per compute
-// unit free, so tracking kernels (of this server or of another server on
-// the same GPU) start within about a slice.  Slicing changes no result bit.
+// one after the other on a grid that leaves the room of two four-wavefront
+// workgroups per compute unit free, so tracking kernels (of this server or of
+// another server on the same GPU) start within about a slice.  Slicing changes no result bit.
 // The two class streams are shared by every server of a device (one per
 // map, say): a process then uses two hardware queues for serving, so a
 // tracking stream never shares a queue with a bulk one.
@@ -151,7 +151,7 @@ struct tsl_server {
     Slot slots[kClasses * kMaxInflight];
     hipStream_t stream[kClasses] = {nullptr, nullptr};
     uint64_t slice_pairs = kDefaultSlicePairs;  // bulk evaluation pairs per launch (0: no slicing)
-    uint32_t reserved_per_cu = 2;  // workgroup slots per CU a sliced bulk evaluation leaves to the other class
+    uint32_t reserved_per_cu = 2;  // four-wavefront workgroups per CU a sliced bulk evaluation leaves room for
     std::thread worker;
     std::atomic<bool> stop{false};
     bool stopped = false;          // worker: stop requested and nothing left (worker thread only)
