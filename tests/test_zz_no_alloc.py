@@ -155,3 +155,41 @@ def test_noalloc_at_the_edges_of_the_spatial_order(tsl, room, P, N):
     assert rc == 0, tsl._lib.lib.tsl_last_error()
     want = ev.evaluate_raw(parts, pts, room.tf)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def test_noalloc_captured_in_spatial_order(tsl, room):
+    """A captured call in spatial order (36 million pairs): every replay sees
+    the particles of its own time, with eager calls between the replays."""
+    torch = pytest.importorskip("torch")
+    from tsdf_localization_amd._lib import check, lib
+    rng = np.random.default_rng(7)
+    P, N = 9000, 4000
+    pts = np.resize(room.points, (N, 3)) + rng.normal(0, 0.01, (N, 3)).astype(np.float32)
+    sets = []
+    for _ in range(3):
+        parts = np.resize(room.particles, (P, 7)).copy()
+        parts[:, :3] += rng.normal(0, 0.5, (P, 3)).astype(np.float32)
+        sets.append(parts[rng.permutation(P)])
+    ev = tsl.TSDFEvaluator(room.map)
+    d_p, d_pts = torch.from_numpy(sets[0]).cuda(), torch.from_numpy(pts).cuda()
+    d_w = torch.zeros(P, device="cuda")
+    tf = np.ascontiguousarray(room.tf, np.float32)
+
+    def call():
+        check(lib.tsl_evaluate_raw_noalloc(ev.handle, d_p.data_ptr(), P, d_pts.data_ptr(), N,
+                                           ctypes.c_void_p(tf.ctypes.data), d_w.data_ptr(),
+                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for parts in sets + sets[:1]:
+        want = ev.evaluate_raw(parts, pts, room.tf)
+        d_p.copy_(torch.from_numpy(parts))
+        d_w.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(d_w.cpu().numpy().view(np.uint32), want.view(np.uint32))
+        _noalloc(ev, parts[:500], pts[:300], room.tf)  # the scratch holds another call's contents
